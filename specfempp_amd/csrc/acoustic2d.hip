@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "solver2d.hpp"
+#include "tile_entries.hpp"
 
 namespace smx {
 
@@ -165,21 +166,28 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
     s_a[i] = MODE == AC_ASSEMBLE ? A[g] : real(0);
   }
   __syncthreads();
-  // point sources first, in list order: -stf L / kappa
-  if (tid == 0)
-    for (int k = T.src_off; k < T.src_off + T.nsrc; ++k) {
-      const int l = src_li[k], s = src_idx[k];
+  // point sources first, in list order: -stf L / kappa (first wavefront)
+  if (ix == 0 && T.nsrc > 0)
+    for (int k0 = 0; k0 < T.nsrc; k0 += ENTRY_GROUP) {
+      const bool act = k0 + lane < T.nsrc;
+      const int k = T.src_off + (act ? k0 + lane : 0);
+      const int code = src_li[k], s = src_idx[k];
+      const real L = src_L[2 * k], kappa = src_L[2 * k + 1];
       const real f = stf[(size_t(step) * nsrc_total + s) * 2];
-      s_a[l] += (real(-1.0) * f * src_L[2 * k]) / src_L[2 * k + 1];
+      const real t = (real(-1.0) * f * L) / kappa;
+      add_entry_group(act ? code : -1, [&](int l) { s_a[l] += t; });
     }
   // coupling with the solid of a coupled mesh: chi_dd += w (n . u), u the
   // elastic displacement after this step's predictor (coupling_terms/
   // acoustic_elastic.hpp:13-26), entries in tile order
-  if (tid == 0)
-    for (int k = T.cpl_off; k < T.cpl_off + T.ncpl; ++k) {
-      const int g = cpl_g[k];
-      s_a[cpl_li[k]] += cpl_w[3 * k] * (cpl_w[3 * k + 1] * Ue[2 * size_t(g)] +
-                                        cpl_w[3 * k + 2] * Ue[2 * size_t(g) + 1]);
+  if (ix == 0 && T.ncpl > 0)
+    for (int k0 = 0; k0 < T.ncpl; k0 += ENTRY_GROUP) {
+      const bool act = k0 + lane < T.ncpl;
+      const int k = T.cpl_off + (act ? k0 + lane : 0);
+      const int code = cpl_li[k], g = cpl_g[k];
+      const real w = cpl_w[3 * k], n0 = cpl_w[3 * k + 1], n1 = cpl_w[3 * k + 2];
+      const real un = n0 * Ue[2 * size_t(g)] + n1 * Ue[2 * size_t(g) + 1];
+      add_entry_group(act ? code : -1, [&](int l) { s_a[l] += w * un; });
     }
 
   // ---- element potential (column ix, rows 0..4)
@@ -602,7 +610,15 @@ public:
     geom_e_ = upload_real(A.geom_e);
     kmr_ = upload_real(A.kappa_mu_rho);
     sslot_ = upload_raw<int>(A.stacey_slot);
-    src_li_ = upload_raw<int>(A.src_li);
+    {
+      std::vector<int32_t> sc(A.src_li.size()), cc(A.cpl_li.size());
+      for (const TileInfo &t : A.tiles) {
+        entry_codes(A.src_li, t.src_off, t.nsrc, sc);
+        entry_codes(A.cpl_li, t.cpl_off, t.ncpl, cc);
+      }
+      src_li_ = upload_raw<int>(sc);
+      cpl_li_ = upload_raw<int>(cc);
+    }
     src_idx_ = upload_raw<int>(A.src_idx);
     src_L_ = upload_real(A.src_L);
     stf_ = upload_real(A.stf);
@@ -635,7 +651,6 @@ public:
     copy_to(stacey_, st);
     minv_ = alloc<real>(n_);
     part_ = alloc<real>(std::max<size_t>(1, A.sh_list.size()));
-    cpl_li_ = upload_raw<int>(A.cpl_li);
     cpl_g_ = upload_raw<int>(A.cpl_idx);
     cpl_w_ = upload_real(A.cpl_w);
     cout_li_ = upload_raw<int>(A.cout_li);

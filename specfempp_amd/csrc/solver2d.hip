@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "solver2d.hpp"
+#include "tile_entries.hpp"
 
 namespace smx {
 
@@ -309,26 +310,38 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
     s_a[i] = z;
   }
   __syncthreads();
-  // point sources first, in list order (one thread: fixed order)
-  if (tid == 0)
-    for (int k = T.src_off; k < T.src_off + T.nsrc; ++k) {
-      const int l = src_li[k], s = src_idx[k];
-      V2 acc = s_a[l];
-      acc.x += stf[(size_t(step) * nsrc_total + s) * 2 + 0] * src_L[2 * k];
-      acc.y += stf[(size_t(step) * nsrc_total + s) * 2 + 1] * src_L[2 * k + 1];
-      s_a[l] = acc;
+  // point sources first, in list order (first wavefront)
+  if (ix == 0 && T.nsrc > 0)
+    for (int k0 = 0; k0 < T.nsrc; k0 += ENTRY_GROUP) {
+      const bool act = k0 + lane < T.nsrc;
+      const int k = T.src_off + (act ? k0 + lane : 0);
+      const int code = src_li[k], s = src_idx[k];
+      const real Lx = src_L[2 * k], Lz = src_L[2 * k + 1];
+      const real fx = stf[(size_t(step) * nsrc_total + s) * 2 + 0];
+      const real fz = stf[(size_t(step) * nsrc_total + s) * 2 + 1];
+      add_entry_group(act ? code : -1, [&](int l) {
+        V2 acc = s_a[l];
+        acc.x += fx * Lx;
+        acc.y += fz * Lz;
+        s_a[l] = acc;
+      });
     }
   // coupling with the fluid of a coupled mesh: a += (w n) chi_dd, the
   // acoustic acceleration of this step (include/medium/dim2/coupling_terms/
   // elastic_acoustic.hpp:13-26), entries in tile order
-  if (tid == 0)
-    for (int k = T.cpl_off; k < T.cpl_off + T.ncpl; ++k) {
-      const int l = cpl_li[k];
+  if (ix == 0 && T.ncpl > 0)
+    for (int k0 = 0; k0 < T.ncpl; k0 += ENTRY_GROUP) {
+      const bool act = k0 + lane < T.ncpl;
+      const int k = T.cpl_off + (act ? k0 + lane : 0);
+      const int code = cpl_li[k];
+      const real w0 = cpl_w[3 * k], w1 = cpl_w[3 * k + 1];
       const real chi = chi_dd[cpl_k[k]];
-      V2 acc = s_a[l];
-      acc.x += cpl_w[3 * k] * chi;
-      acc.y += cpl_w[3 * k + 1] * chi;
-      s_a[l] = acc;
+      add_entry_group(act ? code : -1, [&](int l) {
+        V2 acc = s_a[l];
+        acc.x += w0 * chi;
+        acc.y += w1 * chi;
+        s_a[l] = acc;
+      });
     }
 
   // ---- element displacement (this thread: column ix, rows 0..4)
@@ -1605,7 +1618,15 @@ public:
     kmr_ = upload_real(A.kappa_mu_rho);
     sslot_ = upload_raw<int>(A.stacey_slot);
     stacey_ = upload_real(A.stacey);
-    src_li_ = upload_raw<int>(A.src_li);
+    {
+      std::vector<int32_t> sc(A.src_li.size()), cc(A.cpl_li.size());
+      for (const TileInfo &t : A.tiles) {
+        entry_codes(A.src_li, t.src_off, t.nsrc, sc);
+        entry_codes(A.cpl_li, t.cpl_off, t.ncpl, cc);
+      }
+      src_li_ = upload_raw<int>(sc);
+      cpl_li_ = upload_raw<int>(cc);
+    }
     src_idx_ = upload_raw<int>(A.src_idx);
     src_L_ = upload_real(A.src_L);
     stf_ = upload_real(A.stf);
@@ -1617,7 +1638,6 @@ public:
     rec_slot_ = upload_raw<int>(A.rec_ispec);
     minv_ = alloc<real>(n2_);
     part_ = alloc<real>(2 * std::max<size_t>(1, A.sh_list.size()));
-    cpl_li_ = upload_raw<int>(A.cpl_li);
     cpl_k_ = upload_raw<int>(A.cpl_idx);
     cpl_w_ = upload_real(A.cpl_w);
     lds_bytes_ = tile_lds_bytes<real>(std::max(1, A.nloc_max));

@@ -250,16 +250,21 @@ __global__ void __launch_bounds__(RW * ELEM_THREADS)
   for (int i = tid; i < T.nround * RW; i += RW * ELEM_THREADS)
     s_slot[i] = round_slots[size_t(T.round_off) * RW + i];
   __syncthreads();
-  // point sources first, in list order (one thread: fixed order)
-  if (MODE != M3_ASSEMBLE && tid == 0)
-    for (int k = T.src_off; k < T.src_off + T.nsrc; ++k) {
-      const int l = tsrc_li[k];
-      const real f = stf[size_t(step) * nsrc + tsrc_id[k]];
+  // point sources first, in list order: a source's 125 entries name distinct
+  // points and are added together, one thread each (one thread for the
+  // whole list: 397 instead of 391 us per step of 48^3 elements, 8 sources)
+  if (MODE != M3_ASSEMBLE)
+    for (int k0 = T.src_off; k0 < T.src_off + T.nsrc; k0 += NPT3) {
+      if (tid < NPT3) {
+        const int k = k0 + tid;
+        const int l = tsrc_li[k];
+        const real f = stf[size_t(step) * nsrc + tsrc_id[k]];
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        s_a[c * nloc_max + l] += tsrc_val[size_t(k) * 3 + c] * f;
+        for (int c = 0; c < 3; ++c)
+          s_a[c * nloc_max + l] += tsrc_val[size_t(k) * 3 + c] * f;
+      }
+      __syncthreads();
     }
-  __syncthreads();
 
   // Rounds are software-pipelined: the displacement, geometry and moduli of
   // round r + 1 are requested while round r computes, and the tile-local
