@@ -31,8 +31,8 @@ HBM_PEAK_GBS = 8000.0
 def tile_kernel_bytes(nspec, layout, nstacey):
     """Algorithmic bytes of one k_tile launch (one time step, FP32):
     * per GLL point of an element a 2-byte tile-local index (50 B/element);
-    * geometry: 5 terms per GLL point (500 B/element), or 5 per element
-      (20 B) in tiles of affine elements;
+    * geometry: the element's 4 control nodes (32 B), from which the kernel
+      forms its terms;
     * moduli (lambda+2mu, mu): per GLL point (200 B/element), or per element
       (8 B) in tiles of element-constant material;
     * per point exclusive to a tile: u, v, 1/M read, u, v written: 40 B;
@@ -40,9 +40,8 @@ def tile_kernel_bytes(nspec, layout, nstacey):
       (a tile's share of a shared point): 8 B written;
     * Stacey elements: 6 boundary terms and the velocity per point,
       32 B x 25 = 800 B per element."""
-    ge = layout.get("geom_elem_elements", 0)
     me = layout.get("mat_elem_elements", 0)
-    per_elem = 50 * nspec + 500 * (nspec - ge) + 20 * ge + 200 * (nspec - me) + 8 * me
+    per_elem = 50 * nspec + 32 * nspec + 200 * (nspec - me) + 8 * me
     return (per_elem + 40 * layout["nexclusive"] + 8 * layout["nshared"]
             + 8 * layout["npartials"] + 800 * nstacey)
 
@@ -51,8 +50,8 @@ def ac_tile_kernel_bytes(nspec, layout, nstacey):
     """Algorithmic bytes of one k_ac_tile launch (acoustic time step, FP32):
     * per element: 2-byte tile-local index per GLL point (50 B), the Stacey
       slot, colour and free-surface mask (9 B);
-    * geometry: 5 terms per GLL point (500 B/element), or 5 per element
-      (20 B) in tiles of affine elements;
+    * geometry: the element's 4 control nodes (32 B), from which the kernel
+      forms its terms;
     * 1/rho per GLL point (100 B/element), or per element (4 B) in tiles of
       element-constant material;
     * per point exclusive to a tile: chi, chi_dot, 1/M read, chi, chi_dot
@@ -61,9 +60,8 @@ def ac_tile_kernel_bytes(nspec, layout, nstacey):
       4 B written;
     * Stacey elements: |n|, edge weight, 1/(rho vp) and the velocity per
       point, 16 B x 25 = 400 B per element."""
-    ge = layout.get("geom_elem_elements", 0)
     me = layout.get("mat_elem_elements", 0)
-    per_elem = 59 * nspec + 500 * (nspec - ge) + 20 * ge + 100 * (nspec - me) + 4 * me
+    per_elem = 59 * nspec + 32 * nspec + 100 * (nspec - me) + 4 * me
     return (per_elem + 20 * layout["nexclusive"] + 4 * layout["nshared"]
             + 4 * layout["npartials"] + 400 * nstacey)
 

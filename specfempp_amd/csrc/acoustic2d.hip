@@ -29,6 +29,7 @@
 #include <string>
 #include <vector>
 
+#include "elem_geom.hpp"
 #include "solver2d.hpp"
 #include "tile_entries.hpp"
 
@@ -53,6 +54,7 @@ constexpr int AC_SEIS_GROUPS = 8;
 template <typename real> struct AcQuad {
   real hp[NGLL][NGLL]; // hp[i][j] = l'_j(xi_i)
   real w[NGLL];
+  Q4Deriv d4;     // of 4-node elements at the GLL nodes
 };
 
 struct AcTypes {
@@ -103,14 +105,16 @@ constexpr int kAcPrefetch = 4;
 // The FP32 time step is held to 8 waves per SIMD (at most 64 VGPRs): its
 // ~15 KB of LDS then lets 6 tiles share a CU (30 waves); measured 124 -> 100
 // us per launch on the 800x600 workload together with the prefetch.
-template <typename real, int MODE>
+template <typename real, int MODE, bool STORED>
 __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
     amdgpu_waves_per_eu(sizeof(real) == 4 && MODE == AC_STEP ? 8 : 1, 8)))
     k_ac_tile(const TileInfo *__restrict__ tiles, int nloc_max,
               const int *__restrict__ sh_list, const uint16_t *__restrict__ lidx,
               const uint8_t *__restrict__ ecolor, int ncolors,
-              const real *__restrict__ geom, const real *__restrict__ mat,
-              const real *__restrict__ geom_e, const real *__restrict__ mat_e,
+              const typename ElemColumn<real, STORED>::T *__restrict__ geo,
+           const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
+              const real *__restrict__ mat,
+              const real *__restrict__ mat_e,
               const int *__restrict__ sslot, const real *__restrict__ stacey,
               const uint32_t *__restrict__ dmask, real *__restrict__ U,
               real *__restrict__ V, real *__restrict__ A,
@@ -140,30 +144,28 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   const int ix = __builtin_amdgcn_readfirstlane(tid >> 6);
   const TileInfo T = tiles[blockIdx.x];
   const int nloc = T.nex + T.nsh;
-  const int slot = blockIdx.x * ELEM_TILE + lane;
+  const size_t slot0 = size_t(blockIdx.x) * ELEM_TILE; // element `lane`: slot0 + lane
   const bool valid = lane < T.ecount;
-  const size_t pld = size_t(NPT) * ld;
   const int step = step_ptr ? *step_ptr : istep;
 
   int li[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz)
-    li[iz] = valid ? int(lidx[size_t(iz * NGLL + ix) * ld + slot]) : 0;
+    li[iz] = valid ? int(at32(lidx + size_t(iz * NGLL + ix) * ld + slot0, lane)) : 0;
 
   // ---- tile points: potential in, accumulator cleared (shared points'
   // global ids at a fixed stride per tile, padded with id 0, so that their
   // loads do not wait on the tile record)
   for (int s = tid; s < sh_stride; s += AC_TILE_THREADS) {
-    const real u = U[sh_pad[size_t(blockIdx.x) * sh_stride + s]];
+    const real u = U[at32(sh_pad + size_t(blockIdx.x) * sh_stride, s)];
     if (s < T.nsh) {
       s_u[T.nex + s] = u;
       s_a[T.nex + s] = real(0);
     }
   }
   for (int i = tid; i < T.nex; i += AC_TILE_THREADS) {
-    const int g = T.ex_off + i;
-    s_u[i] = U[g];
-    s_a[i] = MODE == AC_ASSEMBLE ? A[g] : real(0);
+    s_u[i] = at32(U + T.ex_off, i);
+    s_a[i] = MODE == AC_ASSEMBLE ? at32(A + T.ex_off, i) : real(0);
   }
   __syncthreads();
   // point sources first, in list order: -stf L / kappa (first wavefront)
@@ -206,48 +208,46 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
     real a = 0, b = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      a += q.hp[ix][l] * X(iz * NGLL + l, lane);
-      b += q.hp[iz][l] * c[l];
+      a = fma_(q.hp[ix][l], X(iz * NGLL + l, lane), a);
+      b = fma_(q.hp[iz][l], c[l], b);
     }
     dxi[iz] = a;
     dga[iz] = b;
+    formed(dxi[iz]);
+    formed(dga[iz]);
   }
   __syncthreads(); // the staging area becomes the xi integrand
 
   // ---- T = rho^-1 grad chi, F = J T . dxi/dx (point/stress.hpp:166-183)
-  const bool g_el = (T.flags & TILE_GEOM_ELEM) != 0;
   const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  const size_t gst = g_el ? size_t(ld) : pld;
+  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
   real f1[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
-    const size_t o = size_t(p) * ld + slot;
-    const real *gp = g_el ? geom_e + slot : geom + o;
-    const real xix = gp[0], xiz = gp[gst], gax = gp[2 * gst], gaz = gp[3 * gst],
-               jac = gp[4 * gst];
-    const real rinv = m_el ? mat_e[slot] : mat[o];
-    const real dx = xix * dxi[iz] + gax * dga[iz];
-    const real dz = xiz * dxi[iz] + gaz * dga[iz];
-    const real tx = rinv * dx, tz = rinv * dz;
-    X(p, lane) = jac * (tx * xix + tz * xiz);
-    f1[iz] = jac * (tx * gax + tz * gaz);
+    const PointMap<real> m = col.at(iz);
+    const real rinv = at32((m_el ? mat_e : mat + size_t(p) * ld) + slot0, lane);
+    const real tx = rinv * m.dx(dxi[iz], dga[iz]);
+    const real tz = rinv * m.dz(dxi[iz], dga[iz]);
+    X(p, lane) = m.flux_xi(tx, tz);
+    f1[iz] = m.flux_ga(tx, tz);
   }
   __syncthreads();
 
   // ---- divergence (divergence.hpp:40-74), negation, Stacey, free surface
-  const int bslot = valid ? sslot[slot] : -1;
-  const uint32_t dm = valid ? dmask[slot] : 0u;
+  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
+  const uint32_t dm = valid ? at32(dmask + slot0, lane) : 0u;
   real r[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     real t1 = 0, t2 = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      t1 += X(iz * NGLL + l, lane) * q.hp[l][ix] * q.w[l];
-      t2 += f1[l] * q.hp[l][iz] * q.w[l];
+      t1 = fma_(X(iz * NGLL + l, lane) * q.hp[l][ix], q.w[l], t1);
+      t2 = fma_(f1[l] * q.hp[l][iz], q.w[l], t2);
     }
-    real a = q.w[iz] * t1 + q.w[ix] * t2;
+    real a = fma_(q.w[iz], t1, q.w[ix] * t2);
     a *= real(-1.0);
     const int p = iz * NGLL + ix;
     if (bslot >= 0) {
@@ -272,14 +272,14 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   for (int k = 0; k < kAcPrefetch; ++k) {
     const int i = tid + k * AC_TILE_THREADS;
     if (i < T.nex) {
-      pre_m[k] = Minv[T.ex_off + i];
+      pre_m[k] = at32(Minv + T.ex_off, i);
       if (MODE != AC_ASSEMBLE)
-        pre_v[k] = V[T.ex_off + i];
+        pre_v[k] = at32(V + T.ex_off, i);
     }
   }
 
   // ---- assembly into the tile accumulator, colour by colour
-  const int ecol = valid ? int(ecolor[slot]) : -1;
+  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
   for (int cc = 0; cc < ncolors; ++cc) {
     if (ecol == cc) {
 #pragma unroll
@@ -292,13 +292,12 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   // ---- exclusive points: finish the step; shared points: store partials
   const bool sample = seis_terms != nullptr && (step % nsbs) == 0;
   for (int i = tid, k = 0; i < T.nex; i += AC_TILE_THREADS, ++k) {
-    const int g = T.ex_off + i;
-    const real m = k < kAcPrefetch ? pre_m[k] : Minv[g];
+    const real m = k < kAcPrefetch ? pre_m[k] : at32(Minv + T.ex_off, i);
     if (MODE == AC_ASSEMBLE) {
-      A[g] = s_a[i] * m;
+      at32(A + T.ex_off, i) = s_a[i] * m;
       continue;
     }
-    real v = k < kAcPrefetch ? pre_v[k] : V[g];
+    real v = k < kAcPrefetch ? pre_v[k] : at32(V + T.ex_off, i);
     real a = s_a[i] * m;
     v += dto2 * a;
     if (sample || T.ncout > 0)
@@ -309,15 +308,15 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
       real u = s_u[i];
       u += dt * v + dt2o2 * a;
       v += dto2 * a;
-      U[g] = u;
-      V[g] = v;
+      at32(U + T.ex_off, i) = u;
+      at32(V + T.ex_off, i) = v;
     } else {
-      V[g] = v;
-      A[g] = a;
+      at32(V + T.ex_off, i) = v;
+      at32(A + T.ex_off, i) = a;
     }
   }
   for (int i = T.nex + tid; i < nloc; i += AC_TILE_THREADS)
-    part[T.sh_off + i - T.nex] = s_a[i];
+    at32(part + T.sh_off, i - T.nex) = s_a[i];
   // new accelerations of the tile's exclusive interface points, read by the
   // elastic update of this step
   if (MODE != AC_ASSEMBLE && T.ncout > 0) {
@@ -607,7 +606,11 @@ public:
     ibool_ = upload_raw<int>(A.ibool);
     dmask_ = upload_raw<uint32_t>(A.dmask);
     geom_ = upload_real(A.geom);
-    geom_e_ = upload_real(A.geom_e);
+    stored_ = A.nodes.empty();
+    if (!stored_)
+      nodes_ = upload_raw<float>(A.nodes);
+    else
+      geom_e_ = upload_real(A.geom_e);
     kmr_ = upload_real(A.kappa_mu_rho);
     sslot_ = upload_raw<int>(A.stacey_slot);
     {
@@ -672,9 +675,12 @@ public:
       iface_g_ = upload_raw<int>(ig);
     }
     lds_bytes_ = ac_lds_bytes<real>(std::max(1, A.nloc_max));
-    for (const void *f : {reinterpret_cast<const void *>(&k_ac_tile<real, AC_STEP>),
-                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_FINAL>),
-                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_ASSEMBLE>)})
+    for (const void *f : {reinterpret_cast<const void *>(&k_ac_tile<real, AC_STEP, false>),
+                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_FINAL, false>),
+                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_ASSEMBLE, false>),
+                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_STEP, true>),
+                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_FINAL, true>),
+                          reinterpret_cast<const void *>(&k_ac_tile<real, AC_ASSEMBLE, true>)})
       AC_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  int(lds_bytes_)));
     step_ = alloc<int>(2);
@@ -687,6 +693,7 @@ public:
         size_t(std::max(1, A.nsig)) * ntypes * std::max(1, A.nrec) * 2, 2));
     seis_terms_ = alloc<real>(
         std::max<size_t>(size_t(ntypes) * A.nrec * NPT * 2, 2));
+    quad_.d4 = q4_deriv(A.quad.xi);
     for (int i = 0; i < NGLL; ++i) {
       quad_.w[i] = A.quad.w[i];
       for (int j = 0; j < NGLL; ++j)
@@ -1004,11 +1011,21 @@ private:
   template <int MODE>
   void launch_tiles(Field &F, int istep, int *step_ptr, real *terms,
                     real *part = nullptr) {
+    if (stored_)
+      launch_tiles_as<MODE, true>(F, istep, step_ptr, terms, part);
+    else
+      launch_tiles_as<MODE, false>(F, istep, step_ptr, terms, part);
+  }
+  template <int MODE, bool STORED>
+  void launch_tiles_as(Field &F, int istep, int *step_ptr, real *terms,
+                       real *part) {
     const HostAssembly2D &A = *asm_;
-    k_ac_tile<real, MODE><<<dim3(A.ntiles), dim3(AC_TILE_THREADS), lds_bytes_,
+    k_ac_tile<real, MODE, STORED><<<dim3(A.ntiles), dim3(AC_TILE_THREADS), lds_bytes_,
                             stream_>>>(
-        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, geom_,
-        mat_, geom_e_, mat_e_, sslot_, stacey_, dmask_, F.u, F.v, F.a, minv_,
+        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors,
+        (geometry_source<real, STORED>(nodes_, geom_)),
+        (geometry_source<real, STORED>(nodes_, geom_e_)),
+        mat_, mat_e_, sslot_, stacey_, dmask_, F.u, F.v, F.a, minv_,
         part ? part : part_, src_li_, src_idx_, src_L_, stf_,
         std::max(1, A.nsrc), trec_li_, trec_entry_, rent_w_, rent_h_, terms,
         A.nrec * NPT, types_, int(A.seis_types.size()), A.nsbs, step_ptr, istep,
@@ -1075,13 +1092,15 @@ private:
   uint16_t *lidx_ = nullptr;
   uint8_t *ecolor_ = nullptr;
   uint32_t *dmask_ = nullptr;
+  float *nodes_ = nullptr; // 4-node meshes: control nodes
+  bool stored_ = false; // the mesh has 9-node elements
   // coupled meshes: coupling entries, the elastic displacement they read,
   // and the interface accelerations this solver writes for the elastic one
   int *cpl_li_ = nullptr, *cpl_g_ = nullptr, *cout_li_ = nullptr,
       *cout_k_ = nullptr, *sh_iface_ = nullptr, *iface_g_ = nullptr;
   real *cpl_w_ = nullptr, *chi_dd_ = nullptr;
   const real *ue_ = nullptr;
-  real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *mat_e_ = nullptr,
+  real *geom_ = nullptr, *geom_e_ = nullptr,  *mat_ = nullptr, *mat_e_ = nullptr,
        *kmr_ = nullptr, *stacey_ = nullptr, *src_L_ = nullptr, *stf_ = nullptr,
        *rent_h_ = nullptr, *rent_w_ = nullptr, *minv_ = nullptr,
        *part_ = nullptr, *seis_ = nullptr, *seis_terms_ = nullptr,

@@ -166,6 +166,17 @@ Geo jacobian_at(const float *cx, const float *cz, int ngnod, const float *dxi,
   return g;
 }
 
+// Every slot a unit element (padding slots keep it).
+void identity_nodes(HostAssembly2D &A) {
+  const size_t ld = A.nspec_pad;
+  A.nodes.assign(size_t(8) * ld, 0.0f);
+  for (size_t s = 0; s < ld; ++s) {
+    const float x[8] = {-1, 1, 1, -1, -1, -1, 1, 1};
+    for (int n = 0; n < 8; ++n)
+      A.nodes[n * ld + s] = x[n];
+  }
+}
+
 void location_at(const float *cx, const float *cz, int ngnod, float xi,
                  float ga, float &x, float &z) {
   float N[9];
@@ -619,7 +630,7 @@ void assemble2d(const smx_mesh2d &m, const smx_sources2d &src,
   A.geom_e.assign(size_t(5) * ld, 0.0f);
   A.elem_affine.assign(ld, 0);
   if (ngnod == 4) {
-    A.nodes.assign(size_t(8) * ld, 0.0f);
+    identity_nodes(A);
     for (int e = 0; e < nspec; ++e)
       for (int n = 0; n < 4; ++n) {
         A.nodes[size_t(n) * ld + slot_of[e]] = cx[size_t(e) * 4 + n];
@@ -1411,7 +1422,7 @@ void merge_assemblies(std::vector<HostAssembly2D> &shots, HostAssembly2D &M) {
   for (const auto &S : shots)
     all_q4 = all_q4 && !S.nodes.empty();
   if (all_q4)
-    M.nodes.assign(size_t(8) * ld, 0.0f);
+    identity_nodes(M);
   M.stacey_slot.assign(ld, -1);
   M.stacey.assign(6 * sp, 0.0f);
   M.src_ispec.assign(std::max(1, nsrc), 0);

@@ -63,12 +63,12 @@ struct TileInfo {
 
 // Tile flags: every element of the tile has element-constant geometry
 // (affine element: the five Jacobian terms agree at all 25 points to within
-// FP32 rounding) / element-constant lambda+2mu and mu; the kernels then read
-// the per-element arrays geom_e / mat_e instead of the per-point ones.
+// FP32 rounding), which the kernels then take at the element centre /
+// element-constant lambda+2mu and mu, which they then read per element (mat_e).
 constexpr int32_t TILE_GEOM_ELEM = 1;
 constexpr int32_t TILE_MAT_ELEM = 2;
-// The tile re-forms its per-point geometry from the elements' four control
-// nodes (set by the solver after a bitwise check on the device).
+// The stored per-point geometry of the tile was found equal, bit for bit, to
+// that of the elements' four control nodes (set by the solver's check).
 constexpr int32_t TILE_GEOM_NODES = 4;
 
 struct HostAssembly2D {
@@ -134,7 +134,7 @@ struct HostAssembly2D {
   std::vector<float> geom_e, mat_e;
   std::vector<uint8_t> elem_affine;
   // Control nodes of 4-node elements [8][nspec_pad] (x0..x3, z0..z3), FP32;
-  // empty for 9-node meshes.
+  // empty for 9-node meshes.  Padding slots hold a unit element.
   std::vector<float> nodes;
 
   // Stacey: slot -> boundary slot (-1 if none); per slot [6][NPT][nst_pad]

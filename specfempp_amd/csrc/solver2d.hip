@@ -41,6 +41,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "elem_geom.hpp"
 #include "solver2d.hpp"
 #include "tile_entries.hpp"
 
@@ -60,6 +61,7 @@ template <typename real> struct QuadArgs {
   real hp[NGLL][NGLL]; // hp[i][j] = l'_j(xi_i)
   real w[NGLL];
   float xi[NGLL]; // GLL nodes (FP32, as the host assembly uses them)
+  Q4Deriv d4;     // of 4-node elements at the GLL nodes
 };
 
 // The host assembly's per-point geometry of a 4-node element at (xi, gamma),
@@ -215,21 +217,20 @@ __host__ __device__ constexpr size_t tile_lds_bytes(int nloc_max) {
 // The FP32 time-step variant is held to 7 waves per SIMD (at most 73
 // VGPRs) so that register use does not cut below the 5 tiles per CU the LDS
 // footprint allows.
-// GN: the tiles not flagged element-constant re-form their geometry from
-// the control nodes (instead of reading it per point).
+// STORED: the mesh has 9-node elements, whose geometry is read per point.
 // WPE: if nonzero, the minimum waves per SIMD the compiler must allow (an
 // occupancy variant of the FP32 time-step kernel timed by the autotuner);
 // the arithmetic is the same, only the register allocation changes.
-template <typename real, int MODE, bool GN = false, int WPE = 0>
+template <typename real, int MODE, bool STORED = false, int WPE = 0>
 __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(
-    WPE ? WPE : (sizeof(real) == 4 && MODE == MODE_STEP ? (GN ? 4 : 7) : 1),
+    WPE ? WPE : (sizeof(real) == 4 && MODE == MODE_STEP ? 7 : 1),
     8))) k_tile(const TileInfo *__restrict__ tiles, int nloc_max,
            const int *__restrict__ sh_list, const uint16_t *__restrict__ lidx,
            const uint8_t *__restrict__ ecolor, int ncolors,
-           const real *__restrict__ geom, const real *__restrict__ mat,
-           const real *__restrict__ geom_e, const real *__restrict__ mat_e,
-           const float *__restrict__ nodes,
-           const int *__restrict__ sslot, const real *__restrict__ stacey,
+           const typename ElemColumn<real, STORED>::T *__restrict__ geo,
+           const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
+           const real *__restrict__ mat,
+           const real *__restrict__ mat_e, const int *__restrict__ sslot, const real *__restrict__ stacey,
            real *__restrict__ U, real *__restrict__ V, real *__restrict__ A,
            const real *__restrict__ Minv, real *__restrict__ part,
            const int *__restrict__ src_li, const int *__restrict__ src_idx,
@@ -260,9 +261,8 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   const int tile = blockIdx.x;
   const TileInfo T = tiles[tile];
   const int nloc = T.nex + T.nsh;
-  const int slot = tile * ELEM_TILE + lane;
+  const size_t slot0 = size_t(tile) * ELEM_TILE; // element `lane`: slot0 + lane
   const bool valid = lane < T.ecount;
-  const size_t pld = size_t(NPT) * ld;
   V2 *__restrict__ U2 = reinterpret_cast<V2 *>(U);
   V2 *__restrict__ V2p = reinterpret_cast<V2 *>(V);
   V2 *__restrict__ A2 = reinterpret_cast<V2 *>(A);
@@ -283,14 +283,14 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   int li[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz)
-    li[iz] = valid ? int(lidx[size_t(iz * NGLL + ix) * ld + slot]) : 0;
+    li[iz] = valid ? int(at32(lidx + size_t(iz * NGLL + ix) * ld + slot0, lane)) : 0;
 
   // ---- tile points: displacement in, accumulator cleared.  The global ids
   // of the tile's shared points sit at a fixed stride per tile (sh_pad,
   // padded with id 0), so their displacement loads wait on one load only,
   // not on the tile record as well.
   for (int s = tid; s < sh_stride; s += TILE_THREADS) {
-    const V2 u = U2[sh_pad[size_t(tile) * sh_stride + s]];
+    const V2 u = U2[at32(sh_pad + size_t(tile) * sh_stride, s)];
     if (s < T.nsh) {
       V2 z;
       z.x = 0;
@@ -300,13 +300,12 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
     }
   }
   for (int i = tid; i < T.nex; i += TILE_THREADS) {
-    const int g = T.ex_off + i;
-    s_u[i] = U2[g];
+    s_u[i] = at32(U2 + T.ex_off, i);
     V2 z;
     z.x = 0;
     z.y = 0;
     if (MODE == MODE_ASSEMBLE)
-      z = A2[g];
+      z = at32(A2 + T.ex_off, i);
     s_a[i] = z;
   }
   __syncthreads();
@@ -364,81 +363,79 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
     real a0 = 0, a1 = 0, b0 = 0, b1 = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      a0 += q.hp[ix][l] * X(0, iz * NGLL + l, lane);
-      b0 += q.hp[iz][l] * ux[l];
-      a1 += q.hp[ix][l] * X(1, iz * NGLL + l, lane);
-      b1 += q.hp[iz][l] * uz[l];
+      a0 = fma_(q.hp[ix][l], X(0, iz * NGLL + l, lane), a0);
+      b0 = fma_(q.hp[iz][l], ux[l], b0);
+      a1 = fma_(q.hp[ix][l], X(1, iz * NGLL + l, lane), a1);
+      b1 = fma_(q.hp[iz][l], uz[l], b1);
     }
     dxi_x[iz] = a0;
     dxi_z[iz] = a1;
     dga_x[iz] = b0;
     dga_z[iz] = b1;
+    formed(dxi_x[iz]);
+    formed(dxi_z[iz]);
+    formed(dga_x[iz]);
+    formed(dga_z[iz]);
   }
   __syncthreads(); // the staging area is reused for the xi integrand
 
   // ---- stress (stress.hpp:38-78) and F = J sigma dxi/dx (point/stress.hpp:166-183)
+  // (the FP32 variants other than the plain time step round the x row and szz
+  // in the other order)
+  constexpr bool ZF = sizeof(real) == 8 || MODE == MODE_STEP;
   real f1x[NGLL], f1z[NGLL];
-  // element-constant geometry / moduli of flagged tiles come from the
-  // per-element arrays (uniform choice of base and stride)
-  const bool g_el = (T.flags & TILE_GEOM_ELEM) != 0;
+  // element-constant moduli of flagged tiles come from the per-element
+  // array (uniform choice of base and stride)
   const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  const size_t gst = g_el ? size_t(ld) : pld, mst = m_el ? size_t(ld) : pld;
+  const size_t mst = m_el ? size_t(ld) : size_t(NPT) * ld;
+  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
-    const size_t o = size_t(p) * ld + slot;
-    const real *mp = m_el ? mat_e + slot : mat + o;
-    real xix, xiz, gax, gaz, jac;
-    if (GN && !g_el) {
-      float a0, a1, a2, a3, a4;
-      geom_from_nodes2(nodes + slot, ld, q.xi[ix], q.xi[iz], a0, a1, a2, a3,
-                       a4);
-      xix = a0, xiz = a1, gax = a2, gaz = a3, jac = a4;
-    } else {
-      const real *gp = g_el ? geom_e + slot : geom + o;
-      xix = gp[0], xiz = gp[gst], gax = gp[2 * gst], gaz = gp[3 * gst];
-      jac = gp[4 * gst];
-    }
-    const real l2m = mp[0], mu = mp[mst];
-    const real lam = l2m - real(2.0) * mu;
-    const real du_xx = xix * dxi_x[iz] + gax * dga_x[iz];
-    const real du_xz = xiz * dxi_x[iz] + gaz * dga_x[iz];
-    const real du_zx = xix * dxi_z[iz] + gax * dga_z[iz];
-    const real du_zz = xiz * dxi_z[iz] + gaz * dga_z[iz];
-    const real sxx = l2m * du_xx + lam * du_zz;
-    const real szz = l2m * du_zz + lam * du_xx;
+    const real *mp = (m_el ? mat_e : mat + size_t(p) * ld) + slot0;
+    const PointMap<real> m = col.at(iz);
+    const real l2m = at32(mp, lane), mu = at32(mp + mst, lane);
+    const real lam = fma_(real(-2.0), mu, l2m);
+    const real du_xx = m.dx(dxi_x[iz], dga_x[iz]);
+    const real du_xz = m.dz(dxi_x[iz], dga_x[iz]);
+    const real du_zx = m.dx(dxi_z[iz], dga_z[iz]);
+    const real du_zz = m.dz(dxi_z[iz], dga_z[iz]);
+    const real sxx = fma_(l2m, du_xx, lam * du_zz);
+    const real szz = ZF ? fma_(lam, du_xx, l2m * du_zz)
+                        : fma_(l2m, du_zz, lam * du_xx);
     const real sxz = mu * (du_xz + du_zx);
-    X(0, p, lane) = jac * (sxx * xix + sxz * xiz);
-    X(1, p, lane) = jac * (sxz * xix + szz * xiz);
-    f1x[iz] = jac * (sxx * gax + sxz * gaz);
-    f1z[iz] = jac * (sxz * gax + szz * gaz);
+    X(0, p, lane) = m.template flux_xi<ZF>(sxx, sxz);
+    X(1, p, lane) = m.flux_xi(sxz, szz);
+    f1x[iz] = m.template flux_ga<ZF>(sxx, sxz);
+    f1z[iz] = m.flux_ga(sxz, szz);
   }
   __syncthreads();
 
   // ---- divergence (divergence.hpp:40-74), negation, Stacey (stacey.tpp:46-80)
-  const int bslot = valid ? sslot[slot] : -1;
+  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
   real rx[NGLL], rz[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     real t1x = 0, t1z = 0, t2x = 0, t2z = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      t1x += X(0, iz * NGLL + l, lane) * q.hp[l][ix] * q.w[l];
-      t1z += X(1, iz * NGLL + l, lane) * q.hp[l][ix] * q.w[l];
-      t2x += f1x[l] * q.hp[l][iz] * q.w[l];
-      t2z += f1z[l] * q.hp[l][iz] * q.w[l];
+      t1x = fma_(X(0, iz * NGLL + l, lane) * q.hp[l][ix], q.w[l], t1x);
+      t1z = fma_(X(1, iz * NGLL + l, lane) * q.hp[l][ix], q.w[l], t1z);
+      t2x = fma_(f1x[l] * q.hp[l][iz], q.w[l], t2x);
+      t2z = fma_(f1z[l] * q.hp[l][iz], q.w[l], t2z);
     }
-    real ax = q.w[iz] * t1x + q.w[ix] * t2x;
-    real az = q.w[iz] * t1z + q.w[ix] * t2z;
+    real ax = fma_(q.w[iz], t1x, q.w[ix] * t2x);
+    real az = fma_(q.w[iz], t1z, q.w[ix] * t2z);
     ax *= real(-1.0);
     az *= real(-1.0);
     if (bslot >= 0) {
       const int p = iz * NGLL + ix;
-      const size_t so = size_t(p) * sld + bslot;
+      const real *st = stacey + size_t(p) * sld;
       const size_t sp = size_t(NPT) * sld;
-      const real n0 = stacey[so], n1 = stacey[sp + so],
-                 nrm = stacey[2 * sp + so], wgt = stacey[3 * sp + so],
-                 rvp = stacey[4 * sp + so], rvs = stacey[5 * sp + so];
+      const real n0 = at32(st, bslot), n1 = at32(st + sp, bslot),
+                 nrm = at32(st + 2 * sp, bslot), wgt = at32(st + 3 * sp, bslot),
+                 rvp = at32(st + 4 * sp, bslot), rvs = at32(st + 5 * sp, bslot);
       const int g = li[iz] < T.nex ? T.ex_off + li[iz]
                                    : sh_list[T.sh_off + li[iz] - T.nex];
       const V2 vv = V2p[g];
@@ -460,14 +457,14 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   for (int k = 0; k < kNodePrefetch; ++k) {
     const int i = tid + k * TILE_THREADS;
     if (i < T.nex) {
-      pre_m[k] = M2[T.ex_off + i];
+      pre_m[k] = at32(M2 + T.ex_off, i);
       if (MODE != MODE_ASSEMBLE)
-        pre_v[k] = V2p[T.ex_off + i];
+        pre_v[k] = at32(V2p + T.ex_off, i);
     }
   }
 
   // ---- assembly into the tile accumulator, colour by colour
-  const int ecol = valid ? int(ecolor[slot]) : -1;
+  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
   for (int c = 0; c < ncolors; ++c) {
     if (ecol == c) {
 #pragma unroll
@@ -484,22 +481,21 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   // ---- exclusive points: finish the step; shared points: store partials
   const bool sample = seis_terms != nullptr && (step % nsbs) == 0;
   for (int i = tid, k = 0; i < T.nex; i += TILE_THREADS, ++k) {
-    const int g = T.ex_off + i;
     const V2 acc = s_a[i];
     V2 m, v;
     if (k < kNodePrefetch) {
       m = pre_m[k];
       v = pre_v[k];
     } else {
-      m = M2[g];
+      m = at32(M2 + T.ex_off, i);
       if (MODE != MODE_ASSEMBLE)
-        v = V2p[g];
+        v = at32(V2p + T.ex_off, i);
     }
     if (MODE == MODE_ASSEMBLE) {
       V2 a;
       a.x = acc.x * m.x;
       a.y = acc.y * m.y;
-      A2[g] = a;
+      at32(A2 + T.ex_off, i) = a;
       continue;
     }
     V2 a = acc;
@@ -511,23 +507,23 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
     }
     if (MODE == MODE_STEP || MODE == MODE_RECORD) {
       if (MODE == MODE_RECORD)
-        rec_a[g] = a;
+        at32(rec_a + T.ex_off, i) = a;
       V2 u = s_u[i];
       predict(u.x, v.x, a.x, dt, dto2, dt2o2);
       predict(u.y, v.y, a.y, dt, dto2, dt2o2);
-      U2[g] = u;
-      V2p[g] = v;
+      at32(U2 + T.ex_off, i) = u;
+      at32(V2p + T.ex_off, i) = v;
       if (MODE == MODE_RECORD) {
-        rec_u[g] = u;
-        rec_v[g] = v;
+        at32(rec_u + T.ex_off, i) = u;
+        at32(rec_v + T.ex_off, i) = v;
       }
     } else {
-      V2p[g] = v;
-      A2[g] = a;
+      at32(V2p + T.ex_off, i) = v;
+      at32(A2 + T.ex_off, i) = a;
     }
   }
   for (int i = T.nex + tid; i < nloc; i += TILE_THREADS)
-    P2[T.sh_off + i - T.nex] = s_a[i];
+    at32(P2 + T.sh_off, i - T.nex) = s_a[i];
 
   // ---- receiver terms on exclusive points: h * field at step n
   if (MODE != MODE_ASSEMBLE && sample && T.nrec > 0) {
@@ -806,7 +802,7 @@ __global__ void k_seis_pressure(const real *__restrict__ U,
     const real xix = geom[o], xiz = geom[pld + o], gax = geom[2 * pld + o],
                gaz = geom[3 * pld + o];
     const real l2m = mat[o], mu = mat[pld + o];
-    const real lam = l2m - real(2.0) * mu;
+    const real lam = fma_(real(-2.0), mu, l2m);
     const real du_xx = xix * dxi_x + gax * dga_x;
     const real du_zz = xiz * dxi_z + gaz * dga_z;
     const double coef = double(lam) + (2.0 / 3.0) * double(mu);
@@ -1021,16 +1017,16 @@ __device__ __forceinline__ void adj_inject(V2 &ub, int j,
 // assembled in LDS as in k_tile, gradient-density accumulation from rb and
 // the recorded u~, the Stacey impedance terms, and the node update of the
 // tile's exclusive points; shared points get their partial of -K rb.
-template <typename real, bool GN = false>
+template <typename real, bool STORED = false>
 __global__ void __launch_bounds__(TILE_THREADS)
     k_adj_tile(const TileInfo *__restrict__ tiles, int nloc_max,
                const int *__restrict__ sh_list,
                const uint16_t *__restrict__ lidx,
                const uint8_t *__restrict__ ecolor, int ncolors,
-               const real *__restrict__ geom, const real *__restrict__ mat,
-               const real *__restrict__ geom_e, const real *__restrict__ mat_e,
-               const float *__restrict__ nodes,
-               const int *__restrict__ sslot, const real *__restrict__ stacey,
+               const typename ElemColumn<real, STORED>::T *__restrict__ geo,
+           const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
+           const real *__restrict__ mat,
+               const real *__restrict__ mat_e, const int *__restrict__ sslot, const real *__restrict__ stacey,
                real *__restrict__ RB0, real *__restrict__ RB1,
                real *__restrict__ UB, real *__restrict__ VB,
                const real *__restrict__ Minv, real *__restrict__ part,
@@ -1055,9 +1051,8 @@ __global__ void __launch_bounds__(TILE_THREADS)
   const int tile = blockIdx.x;
   const TileInfo T = tiles[tile];
   const int nloc = T.nex + T.nsh;
-  const int slot = tile * ELEM_TILE + lane;
+  const size_t slot0 = size_t(tile) * ELEM_TILE; // element `lane`: slot0 + lane
   const bool valid = lane < T.ecount;
-  const size_t pld = size_t(NPT) * ld;
   const int step = step_ptr[0];
   if (tile == 0 && tid == 0)
     step_ptr[1] = step; // k_adj_shared reads the step from here
@@ -1076,7 +1071,7 @@ __global__ void __launch_bounds__(TILE_THREADS)
   int li[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz)
-    li[iz] = valid ? int(lidx[size_t(iz * NGLL + ix) * ld + slot]) : 0;
+    li[iz] = valid ? int(at32(lidx + size_t(iz * NGLL + ix) * ld + slot0, lane)) : 0;
 
   for (int i = tid; i < nloc; i += TILE_THREADS) {
     const int g = i < T.nex ? T.ex_off + i : sh_list[T.sh_off + i - T.nex];
@@ -1111,6 +1106,10 @@ __global__ void __launch_bounds__(TILE_THREADS)
     uxi_z[iz] = a1;
     uga_x[iz] = b0;
     uga_z[iz] = b1;
+    formed(uxi_x[iz]);
+    formed(uxi_z[iz]);
+    formed(uga_x[iz]);
+    formed(uga_z[iz]);
   }
   __syncthreads(); // staging reused; s_a holds no u~ reads from here on
   for (int i = tid; i < nloc; i += TILE_THREADS) {
@@ -1135,65 +1134,60 @@ __global__ void __launch_bounds__(TILE_THREADS)
     real a0 = 0, a1 = 0, b0 = 0, b1 = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      a0 += q.hp[ix][l] * X(0, iz * NGLL + l, lane);
-      b0 += q.hp[iz][l] * ux[l];
-      a1 += q.hp[ix][l] * X(1, iz * NGLL + l, lane);
-      b1 += q.hp[iz][l] * uz[l];
+      a0 = fma_(q.hp[ix][l], X(0, iz * NGLL + l, lane), a0);
+      b0 = fma_(q.hp[iz][l], ux[l], b0);
+      a1 = fma_(q.hp[ix][l], X(1, iz * NGLL + l, lane), a1);
+      b1 = fma_(q.hp[iz][l], uz[l], b1);
     }
     dxi_x[iz] = a0;
     dxi_z[iz] = a1;
     dga_x[iz] = b0;
     dga_z[iz] = b1;
+    formed(dxi_x[iz]);
+    formed(dxi_z[iz]);
+    formed(dga_x[iz]);
+    formed(dga_z[iz]);
   }
   __syncthreads();
 
   // ---- gradient densities, stress of rb and the xi integrand
   real f1x[NGLL], f1z[NGLL];
-  // element-constant geometry / moduli of flagged tiles come from the
-  // per-element arrays (uniform choice of base and stride)
-  const bool g_el = (T.flags & TILE_GEOM_ELEM) != 0;
+  // element-constant moduli of flagged tiles come from the per-element
+  // array (uniform choice of base and stride)
   const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  const size_t gst = g_el ? size_t(ld) : pld, mst = m_el ? size_t(ld) : pld;
+  const size_t mst = m_el ? size_t(ld) : size_t(NPT) * ld;
+  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
-    const size_t o = size_t(p) * ld + slot;
-    const real *mp = m_el ? mat_e + slot : mat + o;
-    real xix, xiz, gax, gaz, jac;
-    if (GN && !g_el) {
-      float a0, a1, a2, a3, a4;
-      geom_from_nodes2(nodes + slot, ld, q.xi[ix], q.xi[iz], a0, a1, a2, a3,
-                       a4);
-      xix = a0, xiz = a1, gax = a2, gaz = a3, jac = a4;
-    } else {
-      const real *gp = g_el ? geom_e + slot : geom + o;
-      xix = gp[0], xiz = gp[gst], gax = gp[2 * gst], gaz = gp[3 * gst];
-      jac = gp[4 * gst];
-    }
-    const real l2m = mp[0], mu = mp[mst];
-    const real lam = l2m - real(2.0) * mu;
-    const real du_xx = xix * dxi_x[iz] + gax * dga_x[iz];
-    const real du_xz = xiz * dxi_x[iz] + gaz * dga_x[iz];
-    const real du_zx = xix * dxi_z[iz] + gax * dga_z[iz];
-    const real du_zz = xiz * dxi_z[iz] + gaz * dga_z[iz];
-    const real dw_xx = xix * uxi_x[iz] + gax * uga_x[iz];
-    const real dw_xz = xiz * uxi_x[iz] + gaz * uga_x[iz];
-    const real dw_zx = xix * uxi_z[iz] + gax * uga_z[iz];
-    const real dw_zz = xiz * uxi_z[iz] + gaz * uga_z[iz];
+    const size_t o = size_t(p) * ld + slot0;
+    const real *mp = m_el ? mat_e + slot0 : mat + o;
+    const PointMap<real> m = col.at(iz);
+    const real l2m = at32(mp, lane), mu = at32(mp + mst, lane);
+    const real lam = fma_(real(-2.0), mu, l2m);
+    const real du_xx = m.dx(dxi_x[iz], dga_x[iz]);
+    const real du_xz = m.dz(dxi_x[iz], dga_x[iz]);
+    const real du_zx = m.dx(dxi_z[iz], dga_z[iz]);
+    const real du_zz = m.dz(dxi_z[iz], dga_z[iz]);
+    const real dw_xx = m.dx(uxi_x[iz], uga_x[iz]);
+    const real dw_xz = m.dz(uxi_x[iz], uga_x[iz]);
+    const real dw_zx = m.dx(uxi_z[iz], uga_z[iz]);
+    const real dw_zz = m.dz(uxi_z[iz], uga_z[iz]);
     if (valid) {
       const real divr = du_xx + du_zz, divw = dw_xx + dw_zz;
       const real er = real(0.5) * (du_xz + du_zx);
       const real ew = real(0.5) * (dw_xz + dw_zx);
-      Gd[o] += divr * divw;
-      Ge[o] += du_xx * dw_xx + du_zz * dw_zz + real(2.0) * er * ew;
+      at32(Gd + o, lane) += divr * divw;
+      at32(Ge + o, lane) += du_xx * dw_xx + du_zz * dw_zz + real(2.0) * er * ew;
     }
-    const real sxx = l2m * du_xx + lam * du_zz;
-    const real szz = l2m * du_zz + lam * du_xx;
+    const real sxx = fma_(l2m, du_xx, lam * du_zz);
+    const real szz = fma_(lam, du_xx, l2m * du_zz);
     const real sxz = mu * (du_xz + du_zx);
-    X(0, p, lane) = jac * (sxx * xix + sxz * xiz);
-    X(1, p, lane) = jac * (sxz * xix + szz * xiz);
-    f1x[iz] = jac * (sxx * gax + sxz * gaz);
-    f1z[iz] = jac * (sxz * gax + szz * gaz);
+    X(0, p, lane) = m.flux_xi(sxx, sxz);
+    X(1, p, lane) = m.flux_xi(sxz, szz);
+    f1x[iz] = m.flux_ga(sxx, sxz);
+    f1z[iz] = m.flux_ga(sxz, szz);
   }
   __syncthreads();
 
@@ -1204,19 +1198,19 @@ __global__ void __launch_bounds__(TILE_THREADS)
     real t1x = 0, t1z = 0, t2x = 0, t2z = 0;
 #pragma unroll
     for (int l = 0; l < NGLL; ++l) {
-      t1x += X(0, iz * NGLL + l, lane) * q.hp[l][ix] * q.w[l];
-      t1z += X(1, iz * NGLL + l, lane) * q.hp[l][ix] * q.w[l];
-      t2x += f1x[l] * q.hp[l][iz] * q.w[l];
-      t2z += f1z[l] * q.hp[l][iz] * q.w[l];
+      t1x = fma_(X(0, iz * NGLL + l, lane) * q.hp[l][ix], q.w[l], t1x);
+      t1z = fma_(X(1, iz * NGLL + l, lane) * q.hp[l][ix], q.w[l], t1z);
+      t2x = fma_(f1x[l] * q.hp[l][iz], q.w[l], t2x);
+      t2z = fma_(f1z[l] * q.hp[l][iz], q.w[l], t2z);
     }
-    real ax = q.w[iz] * t1x + q.w[ix] * t2x;
-    real az = q.w[iz] * t1z + q.w[ix] * t2z;
+    real ax = fma_(q.w[iz], t1x, q.w[ix] * t2x);
+    real az = fma_(q.w[iz], t1z, q.w[ix] * t2z);
     rx[iz] = real(-1.0) * ax;
     rz[iz] = real(-1.0) * az;
   }
 
   // ---- Stacey impedance terms at this column's absorbing points
-  const int bslot = valid ? sslot[slot] : -1;
+  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
   if (bslot >= 0) {
     const size_t sp = size_t(NPT) * sld;
 #pragma unroll
@@ -1248,7 +1242,7 @@ __global__ void __launch_bounds__(TILE_THREADS)
   }
 
   // ---- assembly into the tile accumulator, colour by colour
-  const int ecol = valid ? int(ecolor[slot]) : -1;
+  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
   for (int c = 0; c < ncolors; ++c) {
     if (ecol == c) {
 #pragma unroll
@@ -1274,33 +1268,31 @@ __global__ void __launch_bounds__(TILE_THREADS)
     for (int k = 0; k < kAdjFin; ++k) {
       const int i = i0 + k * TILE_THREADS;
       if (i < T.nex) {
-        const int g = T.ex_off + i;
-        a[k] = At[g];
-        rr[k] = R[g];
-        ub[k] = UB2[g];
-        vb[k] = VB2[g];
-        m[k] = M2[g];
-        bi[k] = bidx[g];
+        a[k] = at32(At + T.ex_off, i);
+        rr[k] = at32(R + T.ex_off, i);
+        ub[k] = at32(UB2 + T.ex_off, i);
+        vb[k] = at32(VB2 + T.ex_off, i);
+        m[k] = at32(M2 + T.ex_off, i);
+        bi[k] = at32(bidx + T.ex_off, i);
       }
     }
 #pragma unroll
     for (int k = 0; k < kAdjFin; ++k) {
       const int i = i0 + k * TILE_THREADS;
       if (i < T.nex) {
-        const int g = T.ex_off + i;
         const V2 r = s_r[i];
-        R[g] = rr[k] + (r.x * a[k].x + r.y * a[k].y);
+        at32(R + T.ex_off, i) = rr[k] + (r.x * a[k].x + r.y * a[k].y);
         V2 rbn;
         adj_finish<real>(s_a[i], r, ub[k], vb[k], m[k], bi[k], bsum, dt, dto2,
                          dt2o2, rbn);
-        UB2[g] = ub[k];
-        VB2[g] = vb[k];
-        RBn[g] = rbn;
+        at32(UB2 + T.ex_off, i) = ub[k];
+        at32(VB2 + T.ex_off, i) = vb[k];
+        at32(RBn + T.ex_off, i) = rbn;
       }
     }
   }
   for (int i = T.nex + tid; i < nloc; i += TILE_THREADS)
-    P2[T.sh_off + i - T.nex] = s_a[i];
+    at32(P2 + T.sh_off, i - T.nex) = s_a[i];
 }
 
 // Shared points of adjoint step k: partial sums in tile order and the node
@@ -1613,7 +1605,11 @@ public:
     ibool_ = upload_raw<int>(A.ibool);
     geom_ = upload_real(A.geom);
     mat_ = upload_real(A.lam2mu_mu);
-    geom_e_ = upload_real(A.geom_e);
+    stored_ = A.nodes.empty();
+    if (!stored_)
+      nodes_ = upload_raw<float>(A.nodes);
+    else
+      geom_e_ = upload_real(A.geom_e);
     mat_e_ = alloc<real>(A.mat_e.size());
     kmr_ = upload_real(A.kappa_mu_rho);
     sslot_ = upload_raw<int>(A.stacey_slot);
@@ -1665,7 +1661,9 @@ public:
                                   int(lds_bytes_)));
     if constexpr (std::is_same<real, float>::value)
       for (const void *f : {reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 6>),
-                            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 8>)})
+                            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 8>),
+                            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, true, 6>),
+                            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, true, 8>)})
         SMX_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     int(lds_bytes_)));
     // [0] step of the forward / recompute, [1] its copy for k_shared,
@@ -1677,6 +1675,7 @@ public:
     seis_ = alloc<real>(std::max<size_t>(nseis, 2));
     seis_terms_ = alloc<real>(
         std::max<size_t>(size_t(ntypes) * A.nrec * NPT * 2, 2));
+    quad_.d4 = q4_deriv(A.quad.xi);
     for (int i = 0; i < NGLL; ++i) {
       quad_.w[i] = A.quad.w[i];
       quad_.xi[i] = A.quad.xi[i];
@@ -1701,7 +1700,7 @@ public:
     field(SMX_FIELD_FORWARD);
     upload_material();
     if (nodes_geometry && !A.nodes.empty())
-      try_geometry_from_nodes();
+      check_geometry_from_nodes();
     SMX_HIP(hipStreamSynchronize(stream_));
   }
 
@@ -2362,18 +2361,27 @@ private:
   void launch_tiles(real *U, real *V, real *Aout, real *part, int istep,
                     int *step_ptr, real *terms = nullptr,
                     real *rec = nullptr) {
+    if (stored_)
+      launch_tiles_as<MODE, true>(U, V, Aout, part, istep, step_ptr, terms, rec);
+    else
+      launch_tiles_as<MODE, false>(U, V, Aout, part, istep, step_ptr, terms, rec);
+  }
+  template <int MODE, bool STORED>
+  void launch_tiles_as(real *U, real *V, real *Aout, real *part, int istep,
+                       int *step_ptr, real *terms, real *rec) {
     const HostAssembly2D &A = *asm_;
     const int ntypes = int(A.seis_types.size());
-    auto kern = gmode_ == 2 ? &k_tile<real, MODE, true> : &k_tile<real, MODE, false>;
+    auto kern = &k_tile<real, MODE, STORED>;
     if constexpr (MODE == MODE_STEP && std::is_same<real, float>::value) {
-      if (gmode_ != 2 && wpe_ == 6)
-        kern = &k_tile<real, MODE, false, 6>;
-      else if (gmode_ != 2 && wpe_ == 8)
-        kern = &k_tile<real, MODE, false, 8>;
+      if (wpe_ == 6)
+        kern = &k_tile<real, MODE, STORED, 6>;
+      else if (wpe_ == 8)
+        kern = &k_tile<real, MODE, STORED, 8>;
     }
     kern<<<dim3(A.ntiles), dim3(TILE_THREADS), lds_bytes_, stream_>>>(
-        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, geom_,
-        mat_, geom_e_, mat_e_, nodes_, sslot_, stacey_, U, V, Aout, minv_,
+        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, (geometry_source<real, STORED>(nodes_, geom_)),
+        (geometry_source<real, STORED>(nodes_, geom_e_)),
+        mat_, mat_e_, sslot_, stacey_, U, V, Aout, minv_,
         part ? part : part_, src_li_,
         src_idx_, src_L_, stf_, std::max(1, A.nsrc), trec_li_, trec_entry_,
         rent_h_, terms, A.nrec * NPT, stypes_, ntypes, A.nsbs, step_ptr, istep,
@@ -2413,16 +2421,13 @@ private:
   }
   long rec_stride() const { return long(n2_ * sizeof(real)); }
 
-  // Tiles whose geometry is not element-constant re-form it from the control
-  // nodes when the device reproduces every stored per-point value bit for bit
-  // (checked once here); otherwise they keep reading the stored values.
-  void try_geometry_from_nodes() {
+  // Checks on the device whether the control nodes reproduce every stored
+  // per-point value bit for bit, and marks the tiles if so.  The steps form
+  // their geometry from the elements' mappings in either case.
+  void check_geometry_from_nodes() {
     HostAssembly2D &A = *asm_;
     const int ld = A.nspec_pad;
     const size_t n = size_t(NPT) * ld;
-    nodes_ = alloc<float>(A.nodes.size());
-    SMX_HIP(hipMemcpyAsync(nodes_, A.nodes.data(), A.nodes.size() * sizeof(float),
-                           hipMemcpyHostToDevice, stream_));
     float *gf = nullptr;
     unsigned char *bad = nullptr;
     SMX_HIP(hipMalloc(&gf, size_t(5) * n * sizeof(float)));
@@ -2490,19 +2495,27 @@ private:
     launch_tiles<MODE_RECORD>(W.u, W.v, W.a, nullptr, 0, step_, nullptr, rec);
     launch_shared<MODE_RECORD>(W.u, W.v, W.a, step_, rec);
   }
-  // One adjoint step reading the record `rec` (device step counter
-  // step_[2]; own partials buffer, so that it may overlap a recompute).
-  void adjoint_step(Field &B, real *rec, hipStream_t st) {
+  template <bool STORED>
+  void launch_adj_tiles(Field &B, real *rec, hipStream_t st) {
     const HostAssembly2D &A = *asm_;
-    auto kern = gmode_ == 2 ? &k_adj_tile<real, true> : &k_adj_tile<real, false>;
-    kern<<<dim3(A.ntiles), dim3(TILE_THREADS), lds_bytes_, st>>>(
-        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, geom_,
-        mat_, geom_e_, mat_e_, nodes_, sslot_, stacey_, rb0_, rb1_, B.u, B.v,
+    k_adj_tile<real, STORED><<<dim3(A.ntiles), dim3(TILE_THREADS), lds_bytes_, st>>>(
+        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, (geometry_source<real, STORED>(nodes_, geom_)),
+        (geometry_source<real, STORED>(nodes_, geom_e_)),
+        mat_, mat_e_, sslot_, stacey_, rb0_, rb1_, B.u, B.v,
         minv_,
         part_adj_, rec,
         rec_stride(), rec_every_, bidx_, bsum_, gd_, ge_, racc_, sp_, ss_,
         step_ + 2, A.nspec_pad, A.nstacey_pad, dt_, dto2_, dt2o2_, quad_);
     SMX_HIP(hipGetLastError());
+  }
+  // One adjoint step reading the record `rec` (device step counter
+  // step_[2]; own partials buffer, so that it may overlap a recompute).
+  void adjoint_step(Field &B, real *rec, hipStream_t st) {
+    const HostAssembly2D &A = *asm_;
+    if (stored_)
+      launch_adj_tiles<true>(B, rec, st);
+    else
+      launch_adj_tiles<false>(B, rec, st);
     const int nex_rin = int(A.rin_excl.size());
     const int n = std::max(1, A.nshared + nex_rin);
     k_adj_shared<real><<<dim3((n + NODE_THREADS - 1) / NODE_THREADS),
@@ -2689,11 +2702,12 @@ private:
   bool host_model_stale_ = false;
   uint16_t *lidx_ = nullptr;
   uint8_t *ecolor_ = nullptr;
-  real *geom_e_ = nullptr, *mat_e_ = nullptr;
-  float *nodes_ = nullptr;
+  real *mat_e_ = nullptr;
+  float *nodes_ = nullptr; // 4-node meshes: control nodes
+  bool stored_ = false; // the mesh has 9-node elements
   int gmode_ = 0;
   long long geom_mismatch_ = 0;
-  real *geom_ = nullptr, *mat_ = nullptr, *kmr_ = nullptr, *stacey_ = nullptr,
+  real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *kmr_ = nullptr, *stacey_ = nullptr,
        *src_L_ = nullptr, *stf_ = nullptr, *rent_h_ = nullptr,
        *minv_ = nullptr, *part_ = nullptr, *seis_ = nullptr,
        *seis_terms_ = nullptr, *scratch_u_ = nullptr, *scratch_v_ = nullptr,
