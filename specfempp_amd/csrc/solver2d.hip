@@ -13,7 +13,8 @@
 //               in the same pass.  For points shared with other tiles the
 //               tile stores its partial sum in a private slot.
 //   k_shared    sums the partials of each shared point in fixed order, then
-//               the same divide / corrector / predictor.
+//               the same divide / corrector / predictor.  Fields that fit the
+//               memory-side cache do this at the start of the next k_tile.
 //   k_seis_fused, k_seismo   compute_seismograms
 //               (include/kokkos_kernels/impl/compute_seismogram.tpp:19-171).
 //   k_predictor, k_corrector newmark predictor / corrector (operator path).
@@ -184,6 +185,19 @@ __device__ __forceinline__ void divide_correct(real &a, real &v, real minv,
   v += dto2 * a;
 }
 
+// The whole finish of a point between two time steps: divide, corrector, next
+// predictor.  Contractions written out, so that a point is advanced alike
+// wherever it is done: exclusive points (k_tile) round dt/2 a before the
+// predictor adds it, shared points fuse it.
+template <bool SHARED, typename real>
+__device__ __forceinline__ void advance_point(real &u, real &v, real a, real dt,
+                                              real dto2, real dt2o2) {
+#pragma clang fp contract(off)
+  v = fma_(dto2, a, v);
+  u = u + fma_(dt2o2, a, dt * v);
+  v = SHARED ? fma_(dto2, a, v) : v + dto2 * a;
+}
+
 // Sum of the tile partials of shared point j, in tile order.
 template <typename V2>
 __device__ __forceinline__ V2 shared_sum(const V2 *__restrict__ part,
@@ -200,6 +214,87 @@ __device__ __forceinline__ V2 shared_sum(const V2 *__restrict__ part,
   }
   return acc;
 }
+
+// ------------------------------------------------------------------------
+// Seismogram sums of one step from the receiver terms that its tile launch
+// wrote: entries on exclusive points (all entries when only displacement and
+// pressure are recorded, rent_shared = -1) are read, entries on shared points
+// are formed from the state entering the step and its tile partials with the
+// arithmetic of the step.  Sum over a receiver's 25 points in fixed order.
+template <typename real> struct SeisIn {
+  const real *u, *v, *minv; // of the shared points: entering the step, 1/M
+  const real *part;         // the step's partials
+  const int *shp_off, *shp_pos, *rent_shared;
+  const real *rent_h, *terms; // [ntypes][nrec * NPT][2]
+  real *out;                  // [nsig][ntypes][nrec][2]
+  SeisTypes types;
+  int nrec, ntypes, nsbs;
+};
+
+// 32 threads per (type, receiver) pair, pairs from pair0: lane p < 25 forms
+// the term of point p, lane 0 then sums the 25 in point order.  s_t: 50 values
+// per 32 threads.
+template <typename real>
+__device__ __forceinline__ void seis_pairs(const SeisIn<real> &in, int pair0,
+                                           real *s_t, int step, real dto2) {
+  using V2 = typename Vec2<real>::T;
+  const int grp = threadIdx.x >> 5, p = threadIdx.x & 31;
+  const int pair = pair0 + grp;
+  const int r = pair % in.nrec, it = pair / in.nrec;
+  // pressure types are written by k_seis_pressure
+  const bool active = it < in.ntypes && p < NPT && in.types.t[it & 3] != 3;
+  if (step % in.nsbs != 0)
+    return;
+  const int nentries = in.nrec * NPT, id = r * NPT + p;
+  s_t += grp * NPT * 2;
+  if (active) {
+    const int j = in.rent_shared[id], type = in.types.t[it];
+    const real h = in.rent_h[id];
+    const V2 t = reinterpret_cast<const V2 *>(in.terms)[size_t(it) * nentries + id];
+    real tx = t.x, tz = t.y;
+    if (j >= 0) {
+      V2 f = reinterpret_cast<const V2 *>(in.u)[j];
+      if (type != 0) {
+        V2 v = reinterpret_cast<const V2 *>(in.v)[j];
+        const V2 m = reinterpret_cast<const V2 *>(in.minv)[j];
+        V2 acc = shared_sum(reinterpret_cast<const V2 *>(in.part), in.shp_off,
+                            in.shp_pos, j);
+        divide_correct(acc.x, v.x, m.x, dto2);
+        divide_correct(acc.y, v.y, m.y, dto2);
+        f = type == 1 ? v : acc;
+      }
+      tx = h * f.x;
+      tz = h * f.y;
+    }
+    s_t[2 * p] = tx;
+    s_t[2 * p + 1] = tz;
+  }
+  __syncthreads();
+  if (active && p == 0) {
+    real sx = 0, sz = 0;
+    for (int k = 0; k < NPT; ++k) {
+      sx += s_t[2 * k];
+      sz += s_t[2 * k + 1];
+    }
+    const int isig = step / in.nsbs;
+    const size_t o = ((size_t(isig) * in.ntypes + it) * in.nrec + r) * 2;
+    in.out[o] = sx;
+    in.out[o + 1] = sz;
+  }
+}
+
+// What a tile launch that also closes the step before it is given: the shared
+// points' state entering that step and its partials, where its owner leaves a
+// point's new state, each shared point's partial slots, and that step's
+// seismograms (formed by the workgroups after the tiles').
+template <typename real> struct Prev {
+  const real *u, *v, *part;
+  real *u_out, *v_out;
+  const int4 *pos; // [ntiles][sh_stride], -1 past the point's last tile
+  SeisIn<real> seis;
+  int *step_next;
+  int nex_total;
+};
 
 // ------------------------------------------------------------------------
 // Dynamic LDS of k_tile: s_u[nloc_max], s_a[nloc_max] (point displacement and
@@ -221,7 +316,12 @@ __host__ __device__ constexpr size_t tile_lds_bytes(int nloc_max) {
 // WPE: if nonzero, the minimum waves per SIMD the compiler must allow (an
 // occupancy variant of the FP32 time-step kernel timed by the autotuner);
 // the arithmetic is the same, only the register allocation changes.
-template <typename real, int MODE, bool STORED = false, int WPE = 0>
+// FIN: the launch first closes the step before it at the tile's shared points
+// (every tile that holds a point sums its partials and advances it, with the
+// same result; the point's first tile stores it), which takes the launch of
+// k_shared out of the step.
+template <typename real, int MODE, bool STORED = false, int WPE = 0,
+          bool FIN = false>
 __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(
     WPE ? WPE : (sizeof(real) == 4 && MODE == MODE_STEP ? 7 : 1),
     8))) k_tile(const TileInfo *__restrict__ tiles, int nloc_max,
@@ -243,7 +343,8 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
            void *__restrict__ rec, long rec_stride, int every,
            const int *__restrict__ cpl_li, const int *__restrict__ cpl_k,
            const real *__restrict__ cpl_w, const real *__restrict__ chi_dd,
-           const int *__restrict__ sh_pad, int sh_stride) {
+           const int *__restrict__ sh_pad, int sh_stride, Prev<real> prev,
+           int ntiles) {
   using V2 = typename Vec2<real>::T;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   V2 *s_u = reinterpret_cast<V2 *>(lds_raw);
@@ -254,11 +355,18 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
     return xr[(c * NPT + p) * ELEM_TILE + l];
   };
   V2 *s_v = reinterpret_cast<V2 *>(xr);
+  // FIN: velocity of the tile's shared points, after the regions above
+  V2 *s_vs = reinterpret_cast<V2 *>(lds_raw + tile_lds_bytes<real>(nloc_max));
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int ix = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile = blockIdx.x;
+  if (FIN && tile >= ntiles) {
+    seis_pairs<real>(prev.seis, (tile - ntiles) * (TILE_THREADS / 32),
+                     reinterpret_cast<real *>(lds_raw), *step_ptr - 1, dto2);
+    return;
+  }
   const TileInfo T = tiles[tile];
   const int nloc = T.nex + T.nsh;
   const size_t slot0 = size_t(tile) * ELEM_TILE; // element `lane`: slot0 + lane
@@ -289,8 +397,47 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   // of the tile's shared points sit at a fixed stride per tile (sh_pad,
   // padded with id 0), so their displacement loads wait on one load only,
   // not on the tile record as well.
+  if (FIN && tile == 0 && tid == 0)
+    *prev.step_next = step + 1;
   for (int s = tid; s < sh_stride; s += TILE_THREADS) {
-    const V2 u = U2[at32(sh_pad + size_t(tile) * sh_stride, s)];
+    const int g = at32(sh_pad + size_t(tile) * sh_stride, s);
+    V2 u;
+    if constexpr (FIN) {
+      // padded entries read the first shared point and are dropped
+      const int4 pos = at32(prev.pos + size_t(tile) * sh_stride, s);
+      const V2 *P = reinterpret_cast<const V2 *>(prev.part);
+      const V2 p0 = P[pos.x], p1 = P[pos.y];
+      V2 p2, p3;
+      p2.x = p2.y = p3.x = p3.y = 0;
+      if (pos.z >= 0)
+        p2 = P[pos.z];
+      if (pos.w >= 0)
+        p3 = P[pos.w];
+      const int j = g - prev.nex_total;
+      u = reinterpret_cast<const V2 *>(prev.u)[j];
+      V2 v = reinterpret_cast<const V2 *>(prev.v)[j];
+      const V2 m = M2[g];
+      real ax = real(0) + p0.x + p1.x, az = real(0) + p0.y + p1.y;
+      if (pos.z >= 0) {
+        ax += p2.x;
+        az += p2.y;
+      }
+      if (pos.w >= 0) {
+        ax += p3.x;
+        az += p3.y;
+      }
+      advance_point<true>(u.x, v.x, ax * m.x, dt, dto2, dt2o2);
+      advance_point<true>(u.y, v.y, az * m.y, dt, dto2, dt2o2);
+      if (s < T.nsh) {
+        s_vs[s] = v;
+        if (pos.x == T.sh_off + s) {
+          reinterpret_cast<V2 *>(prev.u_out)[j] = u;
+          reinterpret_cast<V2 *>(prev.v_out)[j] = v;
+        }
+      }
+    } else {
+      u = U2[g];
+    }
     if (s < T.nsh) {
       V2 z;
       z.x = 0;
@@ -436,9 +583,16 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
       const real n0 = at32(st, bslot), n1 = at32(st + sp, bslot),
                  nrm = at32(st + 2 * sp, bslot), wgt = at32(st + 3 * sp, bslot),
                  rvp = at32(st + 4 * sp, bslot), rvs = at32(st + 5 * sp, bslot);
-      const int g = li[iz] < T.nex ? T.ex_off + li[iz]
-                                   : sh_list[T.sh_off + li[iz] - T.nex];
-      const V2 vv = V2p[g];
+      V2 vv;
+      if (FIN) {
+        if (li[iz] < T.nex)
+          vv = at32(V2p + T.ex_off, li[iz]);
+        else
+          vv = s_vs[li[iz] - T.nex];
+      } else {
+        vv = V2p[li[iz] < T.nex ? T.ex_off + li[iz]
+                                : sh_list[T.sh_off + li[iz] - T.nex]];
+      }
       const real vx = vv.x, vz = vv.y;
       const real vn = vx * n0 + vz * n1;
       const real fx = ((vn * n0 / (nrm * nrm)) * (rvp - rvs)) + vx * rvs;
@@ -499,18 +653,21 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
       continue;
     }
     V2 a = acc;
-    divide_correct(a.x, v.x, m.x, dto2);
-    divide_correct(a.y, v.y, m.y, dto2);
+    a.x *= m.x;
+    a.y *= m.y;
     if (sample) {
       s_a[i] = a;
-      s_v[i] = v;
+      V2 w;
+      w.x = fma_(dto2, a.x, v.x);
+      w.y = fma_(dto2, a.y, v.y);
+      s_v[i] = w;
     }
     if (MODE == MODE_STEP || MODE == MODE_RECORD) {
       if (MODE == MODE_RECORD)
         at32(rec_a + T.ex_off, i) = a;
       V2 u = s_u[i];
-      predict(u.x, v.x, a.x, dt, dto2, dt2o2);
-      predict(u.y, v.y, a.y, dt, dto2, dt2o2);
+      advance_point<false>(u.x, v.x, a.x, dt, dto2, dt2o2);
+      advance_point<false>(u.y, v.y, a.y, dt, dto2, dt2o2);
       at32(U2 + T.ex_off, i) = u;
       at32(V2p + T.ex_off, i) = v;
       if (MODE == MODE_RECORD) {
@@ -518,6 +675,8 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
         at32(rec_v + T.ex_off, i) = v;
       }
     } else {
+      v.x = fma_(dto2, a.x, v.x);
+      v.y = fma_(dto2, a.y, v.y);
       at32(V2p + T.ex_off, i) = v;
       at32(A2 + T.ex_off, i) = a;
     }
@@ -585,12 +744,14 @@ __device__ void seis_sum_block(const SeisSum<real> &ss, int *__restrict__ step_p
 
 // ------------------------------------------------------------------------
 // Points shared between tiles: sum the tiles' partials in fixed order and
-// finish the step as k_tile does for exclusive points.  Thread 0 advances
+// finish the step as k_tile does for exclusive points.  Us, Vs: the shared
+// points' state entering the step (U, V themselves, or the buffer the last
+// tile launch left it in).  Thread 0 advances
 // the device step counter (fused modes), or the seismogram workgroup does
 // when there is one (block 0; the points then start at block 1).
 template <typename real, int MODE>
 __global__ void __launch_bounds__(NODE_THREADS)
-    k_shared(real *__restrict__ U, real *__restrict__ V, real *__restrict__ A,
+    k_shared(const real *Us, const real *Vs, real *U, real *V, real *A,
              const real *__restrict__ Minv, const real *__restrict__ part,
              const int *__restrict__ shp_off, const int *__restrict__ shp_pos,
              int nshared, int nex_total, real dt, real dto2, real dt2o2,
@@ -617,9 +778,9 @@ __global__ void __launch_bounds__(NODE_THREADS)
   }
   if (j >= nshared)
     return;
-  V2 *__restrict__ U2 = reinterpret_cast<V2 *>(U);
-  V2 *__restrict__ V2p = reinterpret_cast<V2 *>(V);
-  V2 *__restrict__ A2 = reinterpret_cast<V2 *>(A);
+  V2 *U2 = reinterpret_cast<V2 *>(U);
+  V2 *V2p = reinterpret_cast<V2 *>(V);
+  V2 *A2 = reinterpret_cast<V2 *>(A);
   const V2 *__restrict__ M2 = reinterpret_cast<const V2 *>(Minv);
   const int g = nex_total + j;
   // the point's own 1/M, v (or a) and u first: they do not wait on the
@@ -630,9 +791,9 @@ __global__ void __launch_bounds__(NODE_THREADS)
   if (MODE == MODE_ASSEMBLE)
     a0 = A2[g];
   else
-    v = V2p[g];
-  if (MODE == MODE_STEP || MODE == MODE_RECORD)
-    u = U2[g];
+    v = reinterpret_cast<const V2 *>(Vs)[j];
+  if (MODE != MODE_ASSEMBLE)
+    u = reinterpret_cast<const V2 *>(Us)[j];
   V2 acc = shared_sum(reinterpret_cast<const V2 *>(part), shp_off, shp_pos, j);
   if (MODE == MODE_ASSEMBLE) {
     V2 a;
@@ -641,14 +802,14 @@ __global__ void __launch_bounds__(NODE_THREADS)
     A2[g] = a;
     return;
   }
-  divide_correct(acc.x, v.x, m.x, dto2);
-  divide_correct(acc.y, v.y, m.y, dto2);
+  acc.x *= m.x;
+  acc.y *= m.y;
   if (MODE == MODE_STEP || MODE == MODE_RECORD) {
     const int jr = MODE == MODE_RECORD ? step % every : 0;
     if (MODE == MODE_RECORD)
       record_ptr<V2>(rec, rec_stride, jr, 2)[g] = acc;
-    predict(u.x, v.x, acc.x, dt, dto2, dt2o2);
-    predict(u.y, v.y, acc.y, dt, dto2, dt2o2);
+    advance_point<true>(u.x, v.x, acc.x, dt, dto2, dt2o2);
+    advance_point<true>(u.y, v.y, acc.y, dt, dto2, dt2o2);
     U2[g] = u;
     V2p[g] = v;
     if (MODE == MODE_RECORD) {
@@ -656,98 +817,22 @@ __global__ void __launch_bounds__(NODE_THREADS)
       record_ptr<V2>(rec, rec_stride, jr + 1, 1)[g] = v;
     }
   } else {
+    v.x = fma_(dto2, acc.x, v.x);
+    v.y = fma_(dto2, acc.y, v.y);
+    U2[g] = u;
     V2p[g] = v;
     A2[g] = acc;
   }
 }
 
 // ------------------------------------------------------------------------
-// Fused-path seismograms, between the tile launch and k_shared: entries the
-// tiles evaluated (those on exclusive points; all of them when only
-// displacement and pressure are recorded, rent_shared = -1) are read from
-// the terms; entries on shared points otherwise are evaluated here from the
-// tile partials with the same divide / corrector arithmetic.  Sum over the
-// 25 points in fixed order.  Runs on every step with velocity or
-// acceleration types, else on the last step of a call only (the other steps
-// sum in k_shared's first workgroup).
+// The seismograms of one step in a launch of their own (the last step of a
+// call, and steps that k_shared closes).
 template <typename real>
-__global__ void k_seis_fused(const real *__restrict__ U,
-                             const real *__restrict__ V,
-                             const real *__restrict__ Minv,
-                             const real *__restrict__ part,
-                             const int *__restrict__ shp_off,
-                             const int *__restrict__ shp_pos,
-                             const int *__restrict__ rent_g,
-                             const int *__restrict__ rent_shared,
-                             const real *__restrict__ rent_h,
-                             const real *__restrict__ seis_terms, int nrec,
-                             SeisTypes types, int ntypes, int nsbs,
-                             const int *__restrict__ step_ptr, real dto2,
-                             real *__restrict__ out) {
-  using V2 = typename Vec2<real>::T;
-  // 32 threads per (type, receiver): lane p < 25 evaluates point p, lane 0
-  // then sums the 25 terms in point order.
-  __shared__ real s_t[SEIS_GROUPS][NPT][2];
-  const int grp = threadIdx.x >> 5, p = threadIdx.x & 31;
-  const int pair = blockIdx.x * SEIS_GROUPS + grp;
-  const int r = pair % nrec, it = pair / nrec;
-  // pressure types are written by k_seis_pressure
-  const bool active = it < ntypes && p < NPT && types.t[it] != 3;
-  // the entry's own data is requested before the step counter is known
-  // (all in bounds for every active lane)
-  const int nentries = nrec * NPT;
-  const int id = r * NPT + p;
-  int j = -1, g = 0;
-  real h = 0, t0 = 0, t1 = 0;
-  if (active) {
-    j = rent_shared[id];
-    g = rent_g[id];
-    h = rent_h[id];
-    t0 = seis_terms[(size_t(it) * nentries + id) * 2];
-    t1 = seis_terms[(size_t(it) * nentries + id) * 2 + 1];
-  }
-  const int step = *step_ptr;
-  if (step % nsbs != 0)
-    return;
-  const int isig = step / nsbs;
-  if (active) {
-    const int type = types.t[it];
-    real tx, tz;
-    if (j < 0) {
-      tx = t0;
-      tz = t1;
-    } else {
-      real fx, fz;
-      if (type == 0) {
-        fx = U[2 * size_t(g)];
-        fz = U[2 * size_t(g) + 1];
-      } else {
-        real vx = V[2 * size_t(g)], vz = V[2 * size_t(g) + 1];
-        const real m0 = Minv[2 * size_t(g)], m1 = Minv[2 * size_t(g) + 1];
-        V2 acc = shared_sum(reinterpret_cast<const V2 *>(part), shp_off,
-                            shp_pos, j);
-        divide_correct(acc.x, vx, m0, dto2);
-        divide_correct(acc.y, vz, m1, dto2);
-        fx = type == 1 ? vx : acc.x;
-        fz = type == 1 ? vz : acc.y;
-      }
-      tx = h * fx;
-      tz = h * fz;
-    }
-    s_t[grp][p][0] = tx;
-    s_t[grp][p][1] = tz;
-  }
-  __syncthreads();
-  if (active && p == 0) {
-    real sx = 0, sz = 0;
-    for (int k = 0; k < NPT; ++k) {
-      sx += s_t[grp][k][0];
-      sz += s_t[grp][k][1];
-    }
-    const size_t o = ((size_t(isig) * ntypes + it) * nrec + r) * 2;
-    out[o] = sx;
-    out[o + 1] = sz;
-  }
+__global__ void __launch_bounds__(32 * SEIS_GROUPS)
+    k_seis_fused(SeisIn<real> in, const int *__restrict__ step_ptr, real dto2) {
+  __shared__ real s_t[SEIS_GROUPS * NPT * 2];
+  seis_pairs<real>(in, blockIdx.x * SEIS_GROUPS, s_t, *step_ptr, dto2);
 }
 
 // Pressure seismograms of elastic P-SV receivers
@@ -894,6 +979,10 @@ __global__ void __launch_bounds__(NODE_THREADS)
 __global__ void k_set_step(int *__restrict__ step_ptr, int value) {
   if (threadIdx.x == 0 && blockIdx.x == 0)
     *step_ptr = value;
+}
+__global__ void k_set_steps(int *__restrict__ step_ptr, int value) {
+  if (threadIdx.x < 2 && blockIdx.x == 0)
+    step_ptr[threadIdx.x] = value + int(threadIdx.x);
 }
 
 // ------------------------------------------------------------------------
@@ -1637,6 +1726,7 @@ public:
     cpl_k_ = upload_raw<int>(A.cpl_idx);
     cpl_w_ = upload_real(A.cpl_w);
     lds_bytes_ = tile_lds_bytes<real>(std::max(1, A.nloc_max));
+    setup_chain();
     SMX_HIP(hipFuncSetAttribute(
         reinterpret_cast<const void *>(&k_tile<real, MODE_STEP>),
         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes_)));
@@ -1668,7 +1758,8 @@ public:
                                     int(lds_bytes_)));
     // [0] step of the forward / recompute, [1] its copy for k_shared,
     // [2] step of the adjoint, [3] its copy for k_adj_shared
-    step_ = alloc<int>(4);
+    // [4], [5] counters of the one-launch steps, by the parity of the step
+    step_ = alloc<int>(6);
     const int ntypes = int(A.seis_types.size());
     const size_t nseis =
         size_t(std::max(1, A.nsig)) * ntypes * std::max(1, A.nrec) * 2;
@@ -1705,7 +1796,8 @@ public:
   }
 
   ~Solver2D() override {
-    drop_graph(graph_, graph_exec_);
+    drop_graph(graph_[0], graph_exec_[0]);
+    drop_graph(graph_[1], graph_exec_[1]);
     for (int b = 0; b < 2; ++b) {
       drop_graph(rec_graph_[b], rec_graph_exec_[b]);
       drop_graph(adj_graph_[b], adj_graph_exec_[b]);
@@ -1755,8 +1847,7 @@ public:
     // run_forward call pays for it.  Under a coupled driver the driver
     // captures both media itself.
     if (!chi_dd_) {
-      build_graph(field(SMX_FIELD_FORWARD));
-      SMX_HIP(hipGraphUpload(graph_exec_, stream_));
+      prepare_graphs(field(SMX_FIELD_FORWARD));
     }
     SMX_HIP(hipStreamSynchronize(stream_));
     initialized_ = true;
@@ -1773,7 +1864,8 @@ public:
     SMX_HIP(hipStreamSynchronize(stream_));
     if (adj_stream_)
       SMX_HIP(hipStreamSynchronize(adj_stream_));
-    drop_graph(graph_, graph_exec_);
+    drop_graph(graph_[0], graph_exec_[0]);
+    drop_graph(graph_[1], graph_exec_[1]);
     for (int b = 0; b < 2; ++b) {
       drop_graph(rec_graph_[b], rec_graph_exec_[b]);
       drop_graph(adj_graph_[b], adj_graph_exec_[b]);
@@ -1781,8 +1873,7 @@ public:
     gsteps_ = graph_steps;
     wpe_ = waves_per_eu;
     if (initialized_) {
-      build_graph(field(SMX_FIELD_FORWARD));
-      SMX_HIP(hipGraphUpload(graph_exec_, stream_));
+      prepare_graphs(field(SMX_FIELD_FORWARD));
       SMX_HIP(hipStreamSynchronize(stream_));
     }
   }
@@ -1865,19 +1956,8 @@ public:
       throw SmxError(SMX_ERR_ARG, "steps outside [0, nstep)");
     Field &F = field(SMX_FIELD_FORWARD);
     SMX_HIP(hipEventRecord(ev0_, stream_));
-    k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, istep0);
-    SMX_HIP(hipGetLastError());
     launch_predictor(F);
-    const int body = nstep - 1; // steps followed by a fused predictor
-    const int reps = body / gsteps_;
-    if (reps > 0) {
-      build_graph(F);
-      for (int r = 0; r < reps; ++r)
-        SMX_HIP(hipGraphLaunch(graph_exec_, stream_));
-    }
-    for (int s = reps * gsteps_; s < body; ++s)
-      fused_step<MODE_STEP>(F);
-    fused_step<MODE_FINAL>(F);
+    forward_steps(F, istep0, nstep, true);
     SMX_HIP(hipEventRecord(ev1_, stream_));
     last_launches_ = nstep;
     have_stats_ = true;
@@ -2100,8 +2180,6 @@ public:
     SMX_HIP(hipEventRecord(adj_ev_[0], stream_));
     for (real *p : {F.u, F.v, F.a}) // from rest
       SMX_HIP(hipMemsetAsync(p, 0, n2_ * sizeof(real), stream_));
-    k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, 0);
-    SMX_HIP(hipGetLastError());
     launch_predictor(F);
     for (int sgm = 0; sgm < nseg; ++sgm) {
       const int k0 = sgm * every, len = std::min(every, A.nstep - k0);
@@ -2110,18 +2188,7 @@ public:
                              hipMemcpyDeviceToDevice, stream_));
       SMX_HIP(hipMemcpyAsync(ck + n2_, F.v, n2_ * sizeof(real),
                              hipMemcpyDeviceToDevice, stream_));
-      const bool last = sgm == nseg - 1;
-      const int body = last ? len - 1 : len;
-      const int reps = body / gsteps_;
-      if (reps > 0) {
-        build_graph(F);
-        for (int r = 0; r < reps; ++r)
-          SMX_HIP(hipGraphLaunch(graph_exec_, stream_));
-      }
-      for (int st = reps * gsteps_; st < body; ++st)
-        fused_step<MODE_STEP>(F);
-      if (last)
-        fused_step<MODE_FINAL>(F);
+      forward_steps(F, k0, len, sgm == nseg - 1);
     }
     SMX_HIP(hipEventRecord(adj_ev_[1], stream_));
     ckpt_every_ = every;
@@ -2366,20 +2433,23 @@ private:
     else
       launch_tiles_as<MODE, false>(U, V, Aout, part, istep, step_ptr, terms, rec);
   }
-  template <int MODE, bool STORED>
+  template <int MODE, bool STORED, bool FIN = false>
   void launch_tiles_as(real *U, real *V, real *Aout, real *part, int istep,
-                       int *step_ptr, real *terms, real *rec) {
+                       int *step_ptr, real *terms, real *rec,
+                       const Prev<real> &prev = {}, int extra = 0) {
     const HostAssembly2D &A = *asm_;
     const int ntypes = int(A.seis_types.size());
-    auto kern = &k_tile<real, MODE, STORED>;
+    auto kern = &k_tile<real, MODE, STORED, 0, FIN>;
     if constexpr (MODE == MODE_STEP && std::is_same<real, float>::value) {
       if (wpe_ == 6)
-        kern = &k_tile<real, MODE, STORED, 6>;
+        kern = &k_tile<real, MODE, STORED, 6, FIN>;
       else if (wpe_ == 8)
-        kern = &k_tile<real, MODE, STORED, 8>;
+        kern = &k_tile<real, MODE, STORED, 8, FIN>;
     }
-    kern<<<dim3(A.ntiles), dim3(TILE_THREADS), lds_bytes_, stream_>>>(
-        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, (geometry_source<real, STORED>(nodes_, geom_)),
+    kern<<<dim3(A.ntiles + extra), dim3(TILE_THREADS),
+           FIN ? lds_fin_ : lds_bytes_, stream_>>>(
+        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors,
+        (geometry_source<real, STORED>(nodes_, geom_)),
         (geometry_source<real, STORED>(nodes_, geom_e_)),
         mat_, mat_e_, sslot_, stacey_, U, V, Aout, minv_,
         part ? part : part_, src_li_,
@@ -2387,7 +2457,7 @@ private:
         rent_h_, terms, A.nrec * NPT, stypes_, ntypes, A.nsbs, step_ptr, istep,
         A.nspec_pad, A.nstacey_pad, dt_, dto2_, dt2o2_, quad_, rec,
         rec_stride(), std::max(1, rec_every_), cpl_li_, cpl_k_, cpl_w_,
-        chi_dd_, sh_pad_, sh_stride_);
+        chi_dd_, sh_pad_, sh_stride_, prev, A.ntiles);
     SMX_HIP(hipGetLastError());
   }
   void launch_pressure(const real *U, const int *step_ptr, int isig) {
@@ -2404,7 +2474,8 @@ private:
   template <int MODE>
   void launch_shared(real *U, real *V, real *Aout, int *step_ptr,
                      real *rec = nullptr, real *part = nullptr,
-                     bool seis = false) {
+                     bool seis = false, const real *us = nullptr,
+                     const real *vs = nullptr) {
     const HostAssembly2D &A = *asm_;
     const int n = std::max(1, A.nshared);
     SeisSum<real> ss{seis_terms_, seis_, stypes_, A.nrec,
@@ -2413,9 +2484,9 @@ private:
       ss.on = 1;
     k_shared<real, MODE><<<dim3((n + NODE_THREADS - 1) / NODE_THREADS + ss.on),
                            dim3(NODE_THREADS), 0, stream_>>>(
-        U, V, Aout, minv_, part ? part : part_, shp_off_, shp_pos_, A.nshared,
-        A.nex_total,
-        dt_, dto2_, dt2o2_, step_ptr, rec, rec_stride(),
+        us ? us : U + 2 * size_t(A.nex_total),
+        vs ? vs : V + 2 * size_t(A.nex_total), U, V, Aout, minv_,
+        part ? part : part_, shp_off_, shp_pos_, A.nshared, A.nex_total, dt_, dto2_, dt2o2_, step_ptr, rec, rec_stride(),
         std::max(1, rec_every_), ss);
     SMX_HIP(hipGetLastError());
   }
@@ -2659,30 +2730,193 @@ private:
     // every term written by the tiles: the sums ride in k_shared's first
     // workgroup on the time steps of the graph
     const bool in_shared = seis && seis_in_tiles_ && MODE == MODE_STEP;
-    if (seis && !in_shared) {
-      const int n = A.nrec * ntypes;
-      k_seis_fused<real><<<dim3((n + SEIS_GROUPS - 1) / SEIS_GROUPS),
-                           dim3(32 * SEIS_GROUPS), 0, stream_>>>(
-          F.u, F.v, minv_, part_, shp_off_, shp_pos_, rent_g_, rent_shared_,
-          rent_h_, seis_terms_, A.nrec, stypes_, ntypes, A.nsbs, step_, dto2_,
-          seis_);
-      SMX_HIP(hipGetLastError());
-    }
+    if (seis && !in_shared)
+      launch_seis(seis_in(F.u + 2 * size_t(A.nex_total),
+                          F.v + 2 * size_t(A.nex_total), part_, seis_terms_),
+                  step_);
     launch_shared<MODE>(F.u, F.v, F.a, step_, nullptr, nullptr, in_shared);
   }
-  void build_graph(Field &F) {
-    capture(graph_, graph_exec_, stream_, [&] {
-      for (int s = 0; s < gsteps_; ++s)
+  SeisIn<real> seis_in(const real *u, const real *v, const real *part,
+                       const real *terms) const {
+    const HostAssembly2D &A = *asm_;
+    return {u, v, minv_ + 2 * size_t(A.nex_total), part, shp_off_, shp_pos_,
+            rent_shared_, rent_h_, terms, seis_, stypes_, A.nrec,
+            int(A.seis_types.size()), A.nsbs};
+  }
+  void launch_seis(const SeisIn<real> &in, const int *step_ptr) {
+    const int n = in.nrec * in.ntypes;
+    k_seis_fused<real><<<dim3((n + SEIS_GROUPS - 1) / SEIS_GROUPS),
+                         dim3(32 * SEIS_GROUPS), 0, stream_>>>(in, step_ptr, dto2_);
+    SMX_HIP(hipGetLastError());
+  }
+
+  // ---- steps of one launch each.  Launch k of a chain closes step k-1 at the
+  // shared points, so partials, the shared points' (u, v), receiver terms and
+  // the step counter alternate between two buffers by the parity of k; launch
+  // 0 starts from the whole state in the field, and k_shared closes the last.
+  // Pressure seismograms and the other medium of a coupled mesh read the
+  // whole displacement between two steps, and the tables hold four tiles per
+  // point: those contexts keep the two launches.  So do fields beyond the
+  // card's 256 MB memory-side cache, where reading every shared point's state
+  // and partials in each of its tiles costs more than the launch: per step,
+  // one launch against two, 20x15 elements 12.1 / 14.6 us, 160x120 14.4 /
+  // 18.8, 320x240 24.1 / 28.3, 680x510 (222 MB) 81.5 / 84.5, but 800x600
+  // (307 MB) 117 / 111; with velocity and acceleration 400x300 35.4 / 44.8.
+  void setup_chain() {
+    const HostAssembly2D &A = *asm_;
+    bool four = A.nshared > 0 && A.cpl_li.empty() &&
+                10 * size_t(A.nglob) * sizeof(real) <= size_t(256) << 20;
+    for (int j = 0; j < A.nshared && four; ++j) {
+      const int n = A.shp_off[j + 1] - A.shp_off[j];
+      four = n >= 2 && n <= 4;
+    }
+    for (int t : A.seis_types)
+      four = four && t != int(SMX_SEIS_PRESSURE);
+    chain_ = four;
+    if (!chain_)
+      return;
+    const size_t n = size_t(A.ntiles) * sh_stride_;
+    // padded entries: the first shared point, whose first slots exist
+    std::vector<int> pad(n, A.nex_total);
+    std::vector<int4> pos(n, make_int4(0, 0, -1, -1));
+    for (int t = 0; t < A.ntiles; ++t)
+      for (int k = 0; k < A.tiles[t].nsh; ++k) {
+        const int g = A.sh_list[A.tiles[t].sh_off + k], j = g - A.nex_total;
+        int q[4] = {0, 0, -1, -1};
+        for (int i = A.shp_off[j]; i < A.shp_off[j + 1]; ++i)
+          q[i - A.shp_off[j]] = A.shp_pos[i];
+        pad[size_t(t) * sh_stride_ + k] = g;
+        pos[size_t(t) * sh_stride_ + k] = make_int4(q[0], q[1], q[2], q[3]);
+      }
+    release(sh_pad_);
+    sh_pad_ = upload_raw<int>(pad);
+    pos4_ = upload_raw<int4>(pos);
+    sh_u_ = alloc<real>(2 * size_t(A.nshared));
+    sh_v_ = alloc<real>(2 * size_t(A.nshared));
+    part2_ = alloc<real>(2 * A.sh_list.size());
+    terms2_ = alloc<real>(std::max<size_t>(
+        A.seis_types.size() * A.nrec * NPT * 2, 2));
+    lds_fin_ = lds_bytes_ + 2 * size_t(sh_stride_) * sizeof(real);
+    std::vector<const void *> kerns{
+        reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 0, true>),
+        reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, true, 0, true>),
+        reinterpret_cast<const void *>(&k_tile<real, MODE_FINAL, false, 0, true>),
+        reinterpret_cast<const void *>(&k_tile<real, MODE_FINAL, true, 0, true>)};
+    if constexpr (std::is_same<real, float>::value)
+      for (const void *f :
+           {reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 6, true>),
+            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, true, 6, true>),
+            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, false, 8, true>),
+            reinterpret_cast<const void *>(&k_tile<real, MODE_STEP, true, 8, true>)})
+        kerns.push_back(f);
+    for (const void *f : kerns)
+      SMX_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(lds_fin_)));
+  }
+  // Buffers of parity q.
+  real *chain_part(int q) { return q ? part2_ : part_; }
+  real *chain_terms(int q) { return q ? terms2_ : seis_terms_; }
+  real *chain_u(Field &F, int q) { return q ? sh_u_ : F.u + 2 * size_t(asm_->nex_total); }
+  real *chain_v(Field &F, int q) { return q ? sh_v_ : F.v + 2 * size_t(asm_->nex_total); }
+  bool records() const { return asm_->nrec > 0 && !asm_->seis_types.empty(); }
+
+  template <int MODE> void chain_launch(Field &F, int k) {
+    const HostAssembly2D &A = *asm_;
+    const int w = k & 1, r = w ^ 1;
+    real *terms = records() ? chain_terms(w) : nullptr;
+    int *count = step_ + 4;
+    if (k == 0) {
+      launch_tiles<MODE>(F.u, F.v, F.a, part_, 0, count, terms);
+      return;
+    }
+    const Prev<real> prev{chain_u(F, r), chain_v(F, r), chain_part(r),
+                          chain_u(F, w), chain_v(F, w), pos4_,
+                          seis_in(chain_u(F, r), chain_v(F, r), chain_part(r),
+                                  chain_terms(r)),
+                          count + r, A.nex_total};
+    const int groups = TILE_THREADS / 32, n = A.nrec * int(A.seis_types.size());
+    const int extra = records() ? (n + groups - 1) / groups : 0;
+    if (stored_)
+      launch_tiles_as<MODE, true, true>(F.u, F.v, F.a, chain_part(w), 0, count + w,
+                                        terms, nullptr, prev, extra);
+    else
+      launch_tiles_as<MODE, false, true>(F.u, F.v, F.a, chain_part(w), 0, count + w,
+                                         terms, nullptr, prev, extra);
+  }
+
+  // Steps istep0 .. istep0 + n - 1 from the predicted state; final: the last
+  // one stores the corrected v and a, else it predicts the next step.
+  void forward_steps(Field &F, int istep0, int n, bool final) {
+    const int body = final ? n - 1 : n;
+    if (!chain_ || chi_dd_) {
+      k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, istep0);
+      SMX_HIP(hipGetLastError());
+      const int reps = body / gsteps_;
+      if (reps > 0) {
+        build_graph(F, 0);
+        for (int r = 0; r < reps; ++r)
+          SMX_HIP(hipGraphLaunch(graph_exec_[0], stream_));
+      }
+      for (int s = reps * gsteps_; s < body; ++s)
         fused_step<MODE_STEP>(F);
+      if (final)
+        fused_step<MODE_FINAL>(F);
+      return;
+    }
+    k_set_steps<<<dim3(1), dim3(64), 0, stream_>>>(step_ + 4, istep0);
+    SMX_HIP(hipGetLastError());
+    int k = 0;
+    if (body > 0)
+      chain_launch<MODE_STEP>(F, k++);
+    while (k > 0 && body - k >= gsteps_) {
+      build_graph(F, k & 1);
+      SMX_HIP(hipGraphLaunch(graph_exec_[k & 1], stream_));
+      k += gsteps_;
+    }
+    while (k < body)
+      chain_launch<MODE_STEP>(F, k++);
+    if (final)
+      chain_launch<MODE_FINAL>(F, k++);
+    const int w = (k - 1) & 1;
+    if (records())
+      launch_seis(seis_in(chain_u(F, w), chain_v(F, w), chain_part(w),
+                          chain_terms(w)),
+                  step_ + 4 + w);
+    if (final)
+      launch_shared<MODE_FINAL>(F.u, F.v, F.a, nullptr, nullptr, chain_part(w),
+                                false, chain_u(F, w), chain_v(F, w));
+    else
+      launch_shared<MODE_STEP>(F.u, F.v, F.a, nullptr, nullptr, chain_part(w),
+                               false, chain_u(F, w), chain_v(F, w));
+  }
+
+  // A replayed piece of gsteps_ steps; of a chain, beginning at a launch k of
+  // parity q.
+  void build_graph(Field &F, int q) {
+    capture(graph_[q], graph_exec_[q], stream_, [&] {
+      for (int s = 0; s < gsteps_; ++s)
+        if (chain_ && !chi_dd_)
+          chain_launch<MODE_STEP>(F, s + 2 - q);
+        else
+          fused_step<MODE_STEP>(F);
     });
+  }
+  // The graphs a run replays: a chain starts its first at k = 1, and meets
+  // both parities when gsteps_ is odd.
+  void prepare_graphs(Field &F) {
+    for (int q = 0; q < 2; ++q)
+      if (chain_ ? (q == 1 || gsteps_ % 2) : q == 0) {
+        build_graph(F, q);
+        SMX_HIP(hipGraphUpload(graph_exec_[q], stream_));
+      }
   }
 
   std::unique_ptr<HostAssembly2D> asm_;
   int device_ = 0;
   hipStream_t stream_ = nullptr;
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
-  hipGraph_t graph_ = nullptr, rec_graph_[2] = {}, adj_graph_[2] = {};
-  hipGraphExec_t graph_exec_ = nullptr, rec_graph_exec_[2] = {},
+  hipGraph_t graph_[2] = {}, rec_graph_[2] = {}, adj_graph_[2] = {};
+  hipGraphExec_t graph_exec_[2] = {}, rec_graph_exec_[2] = {},
                  adj_graph_exec_[2] = {};
   std::vector<void *> allocs_;
   long nglob_pad_ = 0, n2_ = 0;
@@ -2719,6 +2953,11 @@ private:
   real *cpl_w_ = nullptr;
   const real *chi_dd_ = nullptr;
   size_t lds_bytes_ = 0;
+  // one-launch steps (setup_chain): the second buffers and slot tables
+  bool chain_ = false;
+  size_t lds_fin_ = 0;
+  real *sh_u_ = nullptr, *sh_v_ = nullptr, *part2_ = nullptr, *terms2_ = nullptr;
+  int4 *pos4_ = nullptr;
   int *sh_pad_ = nullptr; // [ntiles][sh_stride_] global ids of shared points
   int sh_stride_ = 1;
   Field fields_[3];
