@@ -279,15 +279,6 @@ void validate_tiles(const HostAssembly3D &A) {
 
 } // namespace
 
-void set_model3d(HostAssembly3D &A, const float *kappa, const float *mu,
-                 const float *rho) {
-  if (!kappa || !mu || !rho)
-    throw SmxError(SMX_ERR_ARG, "null model");
-  material3d(A, kappa, mu, rho);
-  impedances3d(A);
-  mass3d(A);
-}
-
 void assemble3d(const smx_mesh3d &m, const smx_sources3d &src,
                 const smx_receivers3d &rec, double dt_in, int nstep,
                 HostAssembly3D &A, const AssemblyOptions3D &opt) {

@@ -111,10 +111,4 @@ void assemble3d(const smx_mesh3d &mesh, const smx_sources3d &sources,
                 HostAssembly3D &out,
                 const AssemblyOptions3D &opt = AssemblyOptions3D());
 
-// Replaces the material ([nspec][125] each, mesh element order) of an
-// assembled problem: moduli, Stacey impedances and mass.  A is unchanged
-// when the model is rejected.
-void set_model3d(HostAssembly3D &A, const float *kappa, const float *mu,
-                 const float *rho);
-
 } // namespace smx

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <limits>
 #include <string>
 #include <vector>
 
@@ -1053,6 +1054,229 @@ __global__ void k3_set_step(int *__restrict__ step_ptr, int value) {
     *step_ptr = value;
 }
 
+// ------------------------------------------------------------------------
+// A new model on the device.  The host recomputed, re-allocated and uploaded
+// every array that follows from (kappa, mu, rho): 16 of the 28 ms of an
+// inversion step on 21x18x16 elements, whose kernels run 6.5 ms.  These passes
+// read each array once and keep the host's operations and orders of summation
+// (no contraction), so the arrays are the same bit for bit.
+
+// flags[0]: smallest mesh element with a non-physical point; flags[1]: set if
+// the moduli vary inside an element.
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_model_check(const float *__restrict__ kappa, const float *__restrict__ mu,
+                   const float *__restrict__ rho, long n, int *__restrict__ flags) {
+#pragma clang fp contract(off)
+  const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n)
+    return;
+  const long e = i / NPT3, o = e * NPT3;
+  const float k = kappa[i], m = mu[i], k0 = kappa[o], m0 = mu[o];
+  if (!(rho[i] > 0) || !(m >= 0) || !(k > 0))
+    atomicMin(&flags[0], int(e));
+  constexpr float c = static_cast<float>(4.0 / 3.0);
+  if (k + c * m != k0 + c * m0 || m != m0)
+    flags[1] = 1;
+}
+
+// The model in slot order, lambda+2mu and mu per point and of point 0.
+template <typename real>
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_model_in(const float *__restrict__ kappa, const float *__restrict__ mu,
+                const float *__restrict__ rho, const int *__restrict__ slot_elem,
+                long n, float *__restrict__ kmr, real *__restrict__ mat_pt,
+                real *__restrict__ mat_el) {
+#pragma clang fp contract(off)
+  const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= n)
+    return;
+  const long s = t / NPT3;
+  const int p = int(t % NPT3);
+  const long i = long(slot_elem[s]) * NPT3 + p;
+  const float k = kappa[i], m = mu[i];
+  kmr[s * 3 * NPT3 + p] = k;
+  kmr[s * 3 * NPT3 + NPT3 + p] = m;
+  kmr[s * 3 * NPT3 + 2 * NPT3 + p] = rho[i];
+  const real L = sizeof(real) == 8 ? real(double(k) + 4.0 / 3.0 * double(m))
+                                   : real(k + static_cast<float>(4.0 / 3.0) * m);
+  mat_pt[s * 2 * NPT3 + p] = L;
+  mat_pt[s * 2 * NPT3 + NPT3 + p] = real(m);
+  if (p == 0) {
+    mat_el[s * 2] = L;
+    mat_el[s * 2 + 1] = real(m);
+  }
+}
+
+// Impedances of the absorbing points ent[k] = slot * 125 + point.
+template <typename real>
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_model_stacey(const uint32_t *__restrict__ ent, uint32_t n,
+                    const int *__restrict__ sslot, const float *__restrict__ kmr,
+                    real *__restrict__ stacey) {
+#pragma clang fp contract(off)
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n)
+    return;
+  const int s = ent[t] / NPT3, p = ent[t] % NPT3;
+  const float *q = kmr + size_t(s) * 3 * NPT3 + p;
+  const float k = q[0], m = q[NPT3], r = q[2 * NPT3];
+  real *st = stacey + size_t(sslot[s]) * 7 * NPT3 + p;
+  if (sizeof(real) == 8) {
+    const double L = double(k) + 4.0 / 3.0 * double(m);
+    st[5 * NPT3] = real(sqrt(L / double(r)) * double(r));
+    st[6 * NPT3] = real(sqrt(double(r) * double(m)));
+  } else {
+    const float L = k + static_cast<float>(4.0 / 3.0) * m;
+    st[5 * NPT3] = real(sqrtf(L / r) * r);
+    st[6 * NPT3] = real(sqrtf(r * m));
+  }
+}
+
+// Mass of each node: its (slot, point) entries in ascending order, summed in
+// double with the Stacey term at v = (-dt/2, -dt/2, -dt/2), and inverted.
+template <typename real>
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_model_mass(const uint32_t *__restrict__ off,
+                  const uint32_t *__restrict__ ent,
+                  int nglob, long npad, const int *__restrict__ sslot,
+                  const real *__restrict__ stacey, const float *__restrict__ kmr,
+                  const float *__restrict__ jac, Quad3<float> q, float dt,
+                  real *__restrict__ minv) {
+#pragma clang fp contract(off)
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= nglob)
+    return;
+  double M[3] = {0, 0, 0};
+  for (uint32_t k = off[g]; k < off[g + 1]; ++k) {
+    const int s = ent[k] / NPT3, p = ent[k] % NPT3;
+    const int iz = p / (NGLL * NGLL), iy = (p / NGLL) % NGLL, ix = p % NGLL;
+    const float f = q.w[iz] * q.w[iy] * q.w[ix] * jac[size_t(s) * NPT3 + p];
+    const float r = kmr[size_t(s) * 3 * NPT3 + 2 * NPT3 + p];
+    const double m0 = sizeof(real) == 8 ? double(r) * double(f) : double(r * f);
+    double add[3] = {m0, m0, m0};
+    const int b = sslot[s];
+    const real *st = stacey + size_t(b < 0 ? 0 : b) * 7 * NPT3 + p;
+    if (b >= 0 && st[4 * NPT3] != real(0)) {
+      const float n[3] = {float(st[0]), float(st[NPT3]), float(st[2 * NPT3])};
+      const float nrm = float(st[3 * NPT3]), w = float(st[4 * NPT3]);
+      const real P = st[5 * NPT3], S = st[6 * NPT3];
+      const float vf = -1.0f * dt * 0.5f;
+      const float vn = vf * n[0] + vf * n[1] + vf * n[2];
+      for (int c = 0; c < 3; ++c)
+        if (sizeof(real) == 8) {
+          const double fc = ((double(vn) * double(n[c]) / (double(nrm) * double(nrm))) *
+                             (double(P) - double(S))) +
+                            double(vf) * double(S);
+          add[c] += -fc * double(nrm) * double(w);
+        } else {
+          const float fc = ((vn * n[c] / (nrm * nrm)) * (float(P) - float(S))) +
+                           vf * float(S);
+          add[c] += double(-1.0f * fc * nrm * w);
+        }
+    }
+    for (int c = 0; c < 3; ++c)
+      M[c] += add[c];
+  }
+  for (int c = 0; c < 3; ++c)
+    minv[c * npad + g] = real(1.0 / M[c]);
+}
+
+// Stacey matrix of each absorbing node (xx, yy, zz, xy, xz, yz), its face
+// points off[j] .. off[j+1] in ascending order.
+template <typename real>
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_model_bmat(const uint32_t *__restrict__ off,
+                  const uint32_t *__restrict__ ent, int nbn,
+                  long nb, const int *__restrict__ sslot,
+                  const real *__restrict__ stacey, real *__restrict__ bmat) {
+#pragma clang fp contract(off)
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= nbn)
+    return;
+  double m[6] = {0, 0, 0, 0, 0, 0};
+  for (uint32_t k = off[j]; k < off[j + 1]; ++k) {
+    const int s = ent[k] / NPT3, p = ent[k] % NPT3;
+    const real *st = stacey + size_t(sslot[s]) * 7 * NPT3 + p;
+    const double n[3] = {double(st[0]), double(st[NPT3]), double(st[2 * NPT3])};
+    const double nrm = double(st[3 * NPT3]), w = double(st[4 * NPT3]);
+    const double P = double(st[5 * NPT3]), S = double(st[6 * NPT3]);
+    const double f = nrm * w, q = (P - S) / (nrm * nrm);
+    m[0] += f * (q * n[0] * n[0] + S);
+    m[1] += f * (q * n[1] * n[1] + S);
+    m[2] += f * (q * n[2] * n[2] + S);
+    m[3] += f * q * n[0] * n[1];
+    m[4] += f * q * n[0] * n[2];
+    m[5] += f * q * n[1] * n[2];
+  }
+  for (int c = 0; c < 6; ++c)
+    bmat[c * nb + j] = real(m[c]);
+}
+
+// d chi / d (kappa, mu, rho) at every point, [3][nspec][125] in mesh element
+// order: wJ and the chain rule in double:
+//   kappa: -wJ Gd,  mu: -wJ (2 Ge - 2/3 Gd),  rho: -wJ (rb . a')_node,
+// plus, at absorbing points, the rho vp / rho vs terms of B and of the
+// Stacey mass, differentiated through rho vp = sqrt(rho (kappa + 4/3 mu))
+// and rho vs = sqrt(rho mu).
+template <typename real>
+__global__ void __launch_bounds__(NODE3_THREADS)
+    k3_gradient_out(const int *__restrict__ slot_elem, const int *__restrict__ ibool,
+                    long n, const int *__restrict__ sslot,
+                    const real *__restrict__ stacey, const float *__restrict__ kmr,
+                    const float *__restrict__ jac, const real *__restrict__ gd,
+                    const real *__restrict__ ge, const real *__restrict__ R,
+                    const int *__restrict__ bidx, const real *__restrict__ t9,
+                    const real *__restrict__ d3, long nb, Quad3<float> q,
+                    double hdt, double *__restrict__ out) {
+#pragma clang fp contract(off)
+  const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n)
+    return;
+  const long s = i / NPT3;
+  const int p = int(i % NPT3);
+  const int iz = p / (NGLL * NGLL), iy = (p / NGLL) % NGLL, ix = p % NGLL;
+  const int g = ibool[i];
+  const double wj = double(q.w[iz]) * q.w[iy] * q.w[ix] * jac[i];
+  double gk = -wj * double(gd[i]);
+  double gm = -wj * (2.0 * double(ge[i]) - 2.0 / 3.0 * double(gd[i]));
+  double gr = -wj * double(R[g]);
+  const int b = sslot[s];
+  const real *st = stacey + size_t(b < 0 ? 0 : b) * 7 * NPT3 + p;
+  if (b >= 0 && st[4 * NPT3] != real(0)) {
+    const double nv[3] = {double(st[0]), double(st[NPT3]), double(st[2 * NPT3])};
+    const double nrm = sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]);
+    const double nh[3] = {nv[0] / nrm, nv[1] / nrm, nv[2] / nrm};
+    const double wt = double(st[4 * NPT3]), s1 = nh[0] + nh[1] + nh[2];
+    const long bi = bidx[g];
+    double rnvn = 0, tr = 0, tp = 0, ts = 0;
+    for (int c = 0; c < 3; ++c) {
+      tr += double(t9[size_t(c * 3 + c) * nb + bi]);
+      for (int d = 0; d < 3; ++d)
+        rnvn += nh[c] * nh[d] * double(t9[size_t(c * 3 + d) * nb + bi]);
+      const double D = double(d3[size_t(c) * nb + bi]);
+      tp += D * nh[c] * s1;
+      ts += D * (1.0 - nh[c] * s1);
+    }
+    const double dP = -(nrm * wt * rnvn + hdt * nrm * wt * tp);
+    const double dS = -(nrm * wt * (tr - rnvn) + hdt * nrm * wt * ts);
+    const float *m3 = kmr + s * 3 * NPT3 + p;
+    const double kk = m3[0], m = m3[NPT3], rh = m3[2 * NPT3];
+    const double L = kk + 4.0 / 3.0 * m;
+    const double P = sqrt(rh * L), S = sqrt(rh * m);
+    gk += dP * rh / (2.0 * P);
+    gm += dP * (4.0 / 3.0) * rh / (2.0 * P);
+    gr += dP * L / (2.0 * P);
+    if (S > 0) {
+      gm += dS * rh / (2.0 * S);
+      gr += dS * m / (2.0 * S);
+    }
+  }
+  const long o = long(slot_elem[s]) * NPT3 + p;
+  out[o] = gk;
+  out[n + o] = gm;
+  out[2 * n + o] = gr;
+}
+
 } // namespace
 
 template <typename real> class Solver3D final : public Solver3DBase {
@@ -1293,13 +1517,59 @@ public:
   }
 
   // ---------------------------------------------------------------- adjoint
+  // The model is checked before anything changes.  Every array is rewritten
+  // in place, so the captured step stays valid unless the moduli change
+  // between per-element and per-point form.  The assembly's host arrays keep
+  // the model they were made with; only the form of the moduli is noted there.
   void set_model(const float *kappa, const float *mu,
                  const float *rho) override {
+    if (!kappa || !mu || !rho)
+      throw SmxError(SMX_ERR_ARG, "null model");
+    HostAssembly3D &A = *asm_;
+    ensure_model_maps();
+    const long n = long(A.nspec) * NPT3;
+    const float *src[3] = {kappa, mu, rho};
+    for (int c = 0; c < 3; ++c)
+      SMX3_HIP(hipMemcpyAsync(model_ + c * n, src[c], n * sizeof(float),
+                              hipMemcpyHostToDevice, stream_));
+    int flags[2] = {std::numeric_limits<int>::max(), 0};
+    SMX3_HIP(hipMemcpyAsync(flags_, flags, sizeof flags, hipMemcpyHostToDevice,
+                            stream_));
+    const dim3 points(unsigned((n + NODE3_THREADS - 1) / NODE3_THREADS));
+    k3_model_check<<<points, NODE3_THREADS, 0, stream_>>>(model_, model_ + n,
+                                                          model_ + 2 * n, n, flags_);
+    SMX3_HIP(hipGetLastError());
+    SMX3_HIP(hipMemcpyAsync(flags, flags_, sizeof flags, hipMemcpyDeviceToHost,
+                            stream_));
     SMX3_HIP(hipStreamSynchronize(stream_));
-    set_model3d(*asm_, kappa, mu, rho);
-    upload_material();
-    build_boundary_nodes();
-    drop_graph(); // the captured launches hold the old material buffers
+    if (flags[0] != std::numeric_limits<int>::max())
+      throw SmxError(SMX_ERR_ARG, "non-physical material at element " +
+                                      std::to_string(flags[0]));
+    A.mat_elem = flags[1] == 0;
+    real *mat = A.mat_elem ? mat_el_ : mat_pt_;
+    if (mat_ != mat) {
+      drop_graph(); // its launches hold the other array
+      if (mat_ != mat_el_ && mat_ != mat_pt_)
+        release(mat_);
+      mat_ = mat;
+    }
+    k3_model_in<real><<<points, NODE3_THREADS, 0, stream_>>>(
+        model_, model_ + n, model_ + 2 * n, slot_elem_, n, kmr_, mat_pt_, mat_el_);
+    SMX3_HIP(hipGetLastError());
+    if (nbp_ > 0) {
+      k3_model_stacey<real><<<dim3((nbp_ + NODE3_THREADS - 1) / NODE3_THREADS),
+                              NODE3_THREADS, 0, stream_>>>(bent_, nbp_, sslot_,
+                                                           kmr_, stacey_);
+      SMX3_HIP(hipGetLastError());
+      k3_model_bmat<real><<<dim3(unsigned((nbn_ + NODE3_THREADS - 1) / NODE3_THREADS)),
+                            NODE3_THREADS, 0, stream_>>>(
+          boff_, bent_, int(nbn_), nbn_alloc_, sslot_, stacey_, bmat_);
+      SMX3_HIP(hipGetLastError());
+    }
+    k3_model_mass<real><<<dim3((A.nglob + NODE3_THREADS - 1) / NODE3_THREADS),
+                          NODE3_THREADS, 0, stream_>>>(
+        moff_, ment_, A.nglob, npad_, sslot_, stacey_, kmr_, jac_, wq_, A.dt, minv_);
+    SMX3_HIP(hipGetLastError());
     ckpt_every_ = 0;
     have_gradient_ = false;
     SMX3_HIP(hipStreamSynchronize(stream_));
@@ -1407,15 +1677,24 @@ public:
     SMX3_HIP(hipEventRecord(adj_ev_[3], stream_));
     have_gradient_ = true;
     have_adj_stats_ = true;
-    grad_valid_ = false;
   }
 
   void get_gradient(double *out) override {
     if (!have_gradient_)
       throw SmxError(SMX_ERR_STATE, "no adjoint run");
-    if (!grad_valid_)
-      finalize_gradient();
-    std::copy(grad_.begin(), grad_.end(), out);
+    const HostAssembly3D &A = *asm_;
+    ensure_model_maps();
+    const long n = long(A.nspec) * NPT3;
+    if (!grad_)
+      grad_ = alloc<double>(3 * size_t(n));
+    k3_gradient_out<real><<<dim3(unsigned((n + NODE3_THREADS - 1) / NODE3_THREADS)),
+                            NODE3_THREADS, 0, stream_>>>(
+        slot_elem_, ibool_, n, sslot_, stacey_, kmr_, jac_, gd_, ge_, racc_, bidx_,
+        t9_, d3_, nbn_alloc_, wq_, 0.5 * double(A.dt), grad_);
+    SMX3_HIP(hipGetLastError());
+    SMX3_HIP(hipMemcpyAsync(out, grad_, 3 * size_t(n) * sizeof(double),
+                            hipMemcpyDeviceToHost, stream_));
+    SMX3_HIP(hipStreamSynchronize(stream_));
   }
 
   void last_adjoint_stats(double *forward_ms, double *adjoint_ms) override {
@@ -1476,7 +1755,6 @@ private:
   // Moduli, Stacey terms (impedances in double for FP64) and inverse mass.
   void upload_material() {
     const HostAssembly3D &A = *asm_;
-    release(mat_);
     mat_ = sizeof(real) == 8 ? upload<real>(A.mat64) : upload<real>(A.mat);
     std::vector<double> st(A.stacey.begin(), A.stacey.end());
     if (sizeof(real) == 8)
@@ -1485,7 +1763,6 @@ private:
           for (int p = 0; p < NPT3; ++p)
             st[(size_t(b) * 7 + 5 + c) * NPT3 + p] =
                 A.stacey64[(size_t(b) * 2 + c) * NPT3 + p];
-    release(stacey_);
     stacey_ = upload<real>(st);
     std::vector<double> mi(size_t(3) * npad_, 1.0);
     for (int c = 0; c < 3; ++c)
@@ -1493,7 +1770,6 @@ private:
         mi[size_t(c) * npad_ + g] = sizeof(real) == 8
                                         ? A.minv64[size_t(c) * A.nglob + g]
                                         : A.minv[size_t(c) * A.nglob + g];
-    release(minv_);
     minv_ = upload<real>(mi);
   }
 
@@ -1540,18 +1816,66 @@ private:
     for (long b = 0; b < nbn_; ++b)
       for (int k = 0; k < 6; ++k)
         bmt[size_t(k) * nb + b] = bm[size_t(b) * 6 + k];
-    bidx_h_ = bidx;
-    release(bidx_);
-    release(bnode_);
-    release(bmat_);
     bidx_ = upload<int>(bidx);
     bnode_ = upload<int>(bnode);
     bmat_ = upload<real>(bmt);
     nbn_alloc_ = nb;
-    // adjoint buffers sized by nb are re-made on the next adjoint run
-    release(t9_);
-    release(d3_);
-    rec_every_ = 0;
+  }
+
+  // What the passes over a new model and the gradient read besides the model:
+  // slot order, Jacobians, each node's (slot, point) entries and each absorbing
+  // node's face points, both ascending; and the arrays they write.
+  void ensure_model_maps() {
+    if (slot_elem_)
+      return;
+    const HostAssembly3D &A = *asm_;
+    const size_t n = size_t(A.nspec) * NPT3;
+    std::vector<uint32_t> off(size_t(A.nglob) + 1, 0), ent(n);
+    for (size_t i = 0; i < n; ++i)
+      ++off[A.ibool[i] + 1];
+    for (int g = 0; g < A.nglob; ++g)
+      off[g + 1] += off[g];
+    std::vector<uint32_t> at(off.begin(), off.end() - 1);
+    for (size_t i = 0; i < n; ++i)
+      ent[at[A.ibool[i]]++] = uint32_t(i);
+    moff_ = upload<uint32_t>(off);
+    ment_ = upload<uint32_t>(ent);
+    // absorbing nodes are numbered by first touch in ascending order
+    std::vector<int> bidx(size_t(A.nglob), -1);
+    std::vector<std::vector<uint32_t>> points;
+    for (int s = 0; s < A.nspec; ++s) {
+      const int b = A.stacey_slot[s];
+      for (int p = 0; b >= 0 && p < NPT3; ++p) {
+        if (A.stacey[(size_t(b) * 7 + 4) * NPT3 + p] == 0.0f)
+          continue;
+        int &j = bidx[A.ibool[size_t(s) * NPT3 + p]];
+        if (j < 0) {
+          j = int(points.size());
+          points.emplace_back();
+        }
+        points[j].push_back(uint32_t(s) * NPT3 + uint32_t(p));
+      }
+    }
+    std::vector<uint32_t> boff(1, 0), bent;
+    for (const auto &l : points) {
+      bent.insert(bent.end(), l.begin(), l.end());
+      boff.push_back(uint32_t(bent.size()));
+    }
+    nbp_ = uint32_t(bent.size());
+    boff_ = upload<uint32_t>(boff);
+    bent_ = upload<uint32_t>(bent);
+    jac_ = upload<float>(A.jac_pt);
+    kmr_ = upload<float>(A.kappa_mu_rho);
+    model_ = alloc<float>(3 * n);
+    mat_pt_ = alloc<real>(2 * n);
+    mat_el_ = alloc<real>(2 * size_t(A.nspec));
+    flags_ = alloc<int>(2);
+    for (int i = 0; i < NGLL; ++i)
+      wq_.w[i] = A.quad.w[i];
+    std::vector<int> slot_elem(A.nspec);
+    for (int e = 0; e < A.nspec; ++e)
+      slot_elem[A.elem_slot[e]] = e;
+    slot_elem_ = upload<int>(slot_elem);
   }
 
   // Device buffers of the adjoint run (kept between runs).
@@ -1707,81 +2031,6 @@ private:
     SMX3_HIP(hipGetLastError());
     k3_step_add<<<1, 64, 0, stream_>>>(adj_step_, -1);
     SMX3_HIP(hipGetLastError());
-  }
-
-  // Chain rule and quadrature on the host, in double:
-  //   kappa: -wJ Gd,  mu: -wJ (2 Ge - 2/3 Gd),  rho: -wJ (rb . a')_node,
-  // plus, at absorbing points, the rho vp / rho vs terms of B and of the
-  // Stacey mass, differentiated through rho vp = sqrt(rho (kappa + 4/3 mu))
-  // and rho vs = sqrt(rho mu).
-  void finalize_gradient() {
-    const HostAssembly3D &A = *asm_;
-    SMX3_HIP(hipStreamSynchronize(stream_));
-    const size_t nloc = size_t(A.nspec) * NPT3;
-    std::vector<real> gd(nloc), ge(nloc), R(static_cast<size_t>(npad_)),
-        t9(size_t(9) * nbn_alloc_), d3(size_t(3) * nbn_alloc_);
-    SMX3_HIP(hipMemcpy(gd.data(), gd_, nloc * sizeof(real), hipMemcpyDeviceToHost));
-    SMX3_HIP(hipMemcpy(ge.data(), ge_, nloc * sizeof(real), hipMemcpyDeviceToHost));
-    SMX3_HIP(hipMemcpy(R.data(), racc_, R.size() * sizeof(real), hipMemcpyDeviceToHost));
-    SMX3_HIP(hipMemcpy(t9.data(), t9_, t9.size() * sizeof(real), hipMemcpyDeviceToHost));
-    SMX3_HIP(hipMemcpy(d3.data(), d3_, d3.size() * sizeof(real), hipMemcpyDeviceToHost));
-    grad_.assign(3 * nloc, 0.0);
-    std::vector<int> slot_elem(A.nspec);
-    for (int e = 0; e < A.nspec; ++e)
-      slot_elem[A.elem_slot[e]] = e;
-    const long nb = nbn_alloc_;
-    const double hdt = 0.5 * double(A.dt);
-    for (int s = 0; s < A.nspec; ++s) {
-      const size_t oe = size_t(slot_elem[s]) * NPT3;
-      const int b = A.stacey_slot[s];
-      for (int iz = 0; iz < NGLL; ++iz)
-        for (int iy = 0; iy < NGLL; ++iy)
-          for (int ix = 0; ix < NGLL; ++ix) {
-            const int p = (iz * NGLL + iy) * NGLL + ix;
-            const size_t i = size_t(s) * NPT3 + p;
-            const int g = A.ibool[i];
-            const double wj = double(A.quad.w[iz]) * A.quad.w[iy] * A.quad.w[ix] *
-                              A.jac_pt[i];
-            double gk = -wj * double(gd[i]);
-            double gm = -wj * (2.0 * double(ge[i]) - 2.0 / 3.0 * double(gd[i]));
-            double gr = -wj * double(R[g]);
-            if (b >= 0 && A.stacey[(size_t(b) * 7 + 4) * NPT3 + p] != 0.0f) {
-              auto at = [&](int c) { return double(A.stacey[(size_t(b) * 7 + c) * NPT3 + p]); };
-              const double nv[3] = {at(0), at(1), at(2)};
-              const double nrm = std::sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]);
-              const double nh[3] = {nv[0] / nrm, nv[1] / nrm, nv[2] / nrm};
-              const double wt = at(4), s1 = nh[0] + nh[1] + nh[2];
-              const long bi = bidx_h_[g];
-              double rnvn = 0, tr = 0, tp = 0, ts = 0;
-              for (int c = 0; c < 3; ++c) {
-                tr += double(t9[size_t(c * 3 + c) * nb + bi]);
-                for (int d = 0; d < 3; ++d)
-                  rnvn += nh[c] * nh[d] * double(t9[size_t(c * 3 + d) * nb + bi]);
-                const double D = d3[size_t(c) * nb + bi];
-                tp += D * nh[c] * s1;
-                ts += D * (1.0 - nh[c] * s1);
-              }
-              const double dP = -(nrm * wt * rnvn + hdt * nrm * wt * tp);
-              const double dS = -(nrm * wt * (tr - rnvn) + hdt * nrm * wt * ts);
-              const size_t o3 = size_t(s) * 3 * NPT3 + p;
-              const double kk = A.kappa_mu_rho[o3], m = A.kappa_mu_rho[o3 + NPT3],
-                           rh = A.kappa_mu_rho[o3 + 2 * NPT3];
-              const double L = kk + 4.0 / 3.0 * m;
-              const double P = std::sqrt(rh * L), S = std::sqrt(rh * m);
-              gk += dP * rh / (2.0 * P);
-              gm += dP * (4.0 / 3.0) * rh / (2.0 * P);
-              gr += dP * L / (2.0 * P);
-              if (S > 0) {
-                gm += dS * rh / (2.0 * S);
-                gr += dS * m / (2.0 * S);
-              }
-            }
-            grad_[oe + p] = gk;
-            grad_[nloc + oe + p] = gm;
-            grad_[2 * nloc + oe + p] = gr;
-          }
-    }
-    grad_valid_ = true;
   }
 
   real *pick(int which) {
@@ -1963,7 +2212,13 @@ private:
   // adjoint
   int ckpt_every_ = 0, ckpt_cap_ = 0, rec_every_ = 0, nrin_ = 0;
   long nbn_ = 0, nbn_alloc_ = 1;
-  std::vector<int> bidx_h_;
+  // device model passes and gradient (ensure_model_maps)
+  int *slot_elem_ = nullptr, *flags_ = nullptr;
+  uint32_t *moff_ = nullptr, *ment_ = nullptr, *boff_ = nullptr, *bent_ = nullptr;
+  uint32_t nbp_ = 0; // absorbing face points
+  float *jac_ = nullptr, *kmr_ = nullptr, *model_ = nullptr;
+  real *mat_pt_ = nullptr, *mat_el_ = nullptr;
+  Quad3<float> wq_{};
   int *bidx_ = nullptr, *bnode_ = nullptr, *adj_step_ = nullptr,
       *rin_node_ = nullptr, *rin_off_ = nullptr, *rin_r_ = nullptr;
   real *ckpt_ = nullptr, *rec_u_ = nullptr, *rec_a_ = nullptr,
@@ -1972,8 +2227,8 @@ private:
        *t9_ = nullptr, *d3_ = nullptr, *bmat_ = nullptr, *gsrc_ = nullptr,
        *rin_h_ = nullptr;
   hipEvent_t adj_ev_[4] = {};
-  bool have_gradient_ = false, have_adj_stats_ = false, grad_valid_ = false;
-  std::vector<double> grad_;
+  bool have_gradient_ = false, have_adj_stats_ = false;
+  double *grad_ = nullptr;
 };
 
 std::unique_ptr<Solver3DBase> make_solver3d(std::unique_ptr<HostAssembly3D> a,
