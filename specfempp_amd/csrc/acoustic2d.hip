@@ -220,8 +220,9 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
 
   // ---- T = rho^-1 grad chi, F = J T . dxi/dx (point/stress.hpp:166-183)
   const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
-                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                               (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  col.open();
   real f1[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {

@@ -122,17 +122,21 @@ template <typename real> struct ElemColumn<real, false> {
   using T = float;
   float x[4], z[4], xg, zg;
   const Q4Deriv &d;
+  const int ix;
   const bool centre;
   __device__ __forceinline__ ElemColumn(const float *__restrict__ geo,
                                         const float *, size_t ld, size_t slot0,
-                                        uint32_t i, int ix, bool centre_,
+                                        uint32_t i, int ix_, bool centre_,
                                         const Q4Deriv &d_)
-      : d(d_), centre(centre_) {
+      : d(d_), ix(ix_), centre(centre_) {
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       x[n] = at32(geo + n * ld + slot0, i);
       z[n] = at32(geo + (4 + n) * ld + slot0, i);
     }
+  }
+  // The column's sums; the constructor only requests the coordinates.
+  __device__ __forceinline__ void open() {
     const float m = centre ? -0.25f : d.m[ix], p = centre ? 0.25f : d.p[ix];
     xg = q4_along_ga(x, m, p);
     zg = q4_along_ga(z, m, p);
@@ -161,6 +165,7 @@ template <typename real> struct ElemColumn<real, true> {
                                         bool centre, const Q4Deriv &)
       : base((centre ? geo_e : geo) + slot0), point(centre ? 0 : ld),
         term(centre ? ld : NPT * ld), i(i_), ix(ix_) {}
+  __device__ __forceinline__ void open() {}
   __device__ __forceinline__ PointMap<real> at(int iz) const {
     const real *p = base + size_t(iz * NGLL + ix) * point;
     return {at32(p, i), at32(p + term, i), at32(p + 2 * term, i),

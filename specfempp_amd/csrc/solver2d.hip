@@ -392,6 +392,21 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz)
     li[iz] = valid ? int(at32(lidx + size_t(iz * NGLL + ix) * ld + slot0, lane)) : 0;
+  // the element's own data, requested with the first loads: a pass over a few
+  // tiles is a chain of waits, and these would add four more to it
+  const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
+  const size_t mst = m_el ? size_t(ld) : size_t(NPT) * ld;
+  real l2ms[NGLL], mus[NGLL];
+#pragma unroll
+  for (int iz = 0; iz < NGLL; ++iz) {
+    const real *mp = (m_el ? mat_e : mat + size_t(iz * NGLL + ix) * ld) + slot0;
+    l2ms[iz] = at32(mp, lane);
+    mus[iz] = at32(mp + mst, lane);
+  }
+  ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                               (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
+  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
 
   // ---- tile points: displacement in, accumulator cleared.  The global ids
   // of the tile's shared points sit at a fixed stride per tile (sh_pad,
@@ -531,18 +546,12 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   // in the other order)
   constexpr bool ZF = sizeof(real) == 8 || MODE == MODE_STEP;
   real f1x[NGLL], f1z[NGLL];
-  // element-constant moduli of flagged tiles come from the per-element
-  // array (uniform choice of base and stride)
-  const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  const size_t mst = m_el ? size_t(ld) : size_t(NPT) * ld;
-  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
-                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  col.open();
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
-    const real *mp = (m_el ? mat_e : mat + size_t(p) * ld) + slot0;
     const PointMap<real> m = col.at(iz);
-    const real l2m = at32(mp, lane), mu = at32(mp + mst, lane);
+    const real l2m = l2ms[iz], mu = mus[iz];
     const real lam = fma_(real(-2.0), mu, l2m);
     const real du_xx = m.dx(dxi_x[iz], dga_x[iz]);
     const real du_xz = m.dz(dxi_x[iz], dga_x[iz]);
@@ -560,7 +569,6 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   __syncthreads();
 
   // ---- divergence (divergence.hpp:40-74), negation, Stacey (stacey.tpp:46-80)
-  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
   real rx[NGLL], rz[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
@@ -618,7 +626,6 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
   }
 
   // ---- assembly into the tile accumulator, colour by colour
-  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
   for (int c = 0; c < ncolors; ++c) {
     if (ecol == c) {
 #pragma unroll
@@ -1245,8 +1252,9 @@ __global__ void __launch_bounds__(TILE_THREADS)
   // array (uniform choice of base and stride)
   const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
   const size_t mst = m_el ? size_t(ld) : size_t(NPT) * ld;
-  const ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
-                                     (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                               (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  col.open();
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
