@@ -152,6 +152,17 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz)
     li[iz] = valid ? int(at32(lidx + size_t(iz * NGLL + ix) * ld + slot0, lane)) : 0;
+  // the element's own data, requested with the first loads
+  const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
+  real rinvs[NGLL];
+#pragma unroll
+  for (int iz = 0; iz < NGLL; ++iz)
+    rinvs[iz] = at32((m_el ? mat_e : mat + size_t(iz * NGLL + ix) * ld) + slot0, lane);
+  ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
+                               (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
+  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
+  const uint32_t dm = valid ? at32(dmask + slot0, lane) : 0u;
+  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
 
   // ---- tile points: potential in, accumulator cleared (shared points'
   // global ids at a fixed stride per tile, padded with id 0, so that their
@@ -219,16 +230,13 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   __syncthreads(); // the staging area becomes the xi integrand
 
   // ---- T = rho^-1 grad chi, F = J T . dxi/dx (point/stress.hpp:166-183)
-  const bool m_el = (T.flags & TILE_MAT_ELEM) != 0;
-  ElemColumn<real, STORED> col(geo, geo_e, size_t(ld), slot0, lane, ix,
-                               (T.flags & TILE_GEOM_ELEM) != 0, q.d4);
   col.open();
   real f1[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
     const int p = iz * NGLL + ix;
     const PointMap<real> m = col.at(iz);
-    const real rinv = at32((m_el ? mat_e : mat + size_t(p) * ld) + slot0, lane);
+    const real rinv = rinvs[iz];
     const real tx = rinv * m.dx(dxi[iz], dga[iz]);
     const real tz = rinv * m.dz(dxi[iz], dga[iz]);
     X(p, lane) = m.flux_xi(tx, tz);
@@ -237,8 +245,6 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   __syncthreads();
 
   // ---- divergence (divergence.hpp:40-74), negation, Stacey, free surface
-  const int bslot = valid ? at32(sslot + slot0, lane) : -1;
-  const uint32_t dm = valid ? at32(dmask + slot0, lane) : 0u;
   real r[NGLL];
 #pragma unroll
   for (int iz = 0; iz < NGLL; ++iz) {
@@ -280,7 +286,6 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   }
 
   // ---- assembly into the tile accumulator, colour by colour
-  const int ecol = valid ? int(at32(ecolor + slot0, lane)) : -1;
   for (int cc = 0; cc < ncolors; ++cc) {
     if (ecol == cc) {
 #pragma unroll
