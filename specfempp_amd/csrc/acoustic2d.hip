@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
               const int *__restrict__ trec_entry,
               const real *__restrict__ rent_w, const real *__restrict__ rent_h,
               real *__restrict__ seis_terms, int nentries, AcTypes types,
-              int ntypes, int nsbs, const int *__restrict__ step_ptr,
+              int ntypes, int nsbs, int *__restrict__ step_ptr,
               int istep, int ld, int sld, real dt, real dto2, real dt2o2,
               AcQuad<real> q, const int *__restrict__ cpl_li,
               const int *__restrict__ cpl_g, const real *__restrict__ cpl_w,
@@ -147,6 +147,8 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
   const size_t slot0 = size_t(blockIdx.x) * ELEM_TILE; // element `lane`: slot0 + lane
   const bool valid = lane < T.ecount;
   const int step = step_ptr ? *step_ptr : istep;
+  if (MODE == AC_STEP && step_ptr && blockIdx.x == 0 && tid == 0)
+    step_ptr[1] = step; // the seismogram workgroups of k_ac_shared read it
 
   int li[NGLL];
 #pragma unroll
@@ -361,6 +363,87 @@ __global__ void k_ac_iface(const real *__restrict__ A,
     chi_dd[k] = A[iface_g[k]];
 }
 
+// Seismogram sums of one step from the receiver terms its tile launch wrote;
+// entries on shared points are finished from the state entering the step and
+// the partials with k_ac_shared's arithmetic; a receiver's 25 terms are summed
+// in point order.
+template <typename real> struct AcSeisIn {
+  const real *u, *v, *minv, *part;
+  const int *shp_off, *shp_pos, *rent_g, *rent_shared;
+  const real *rent_w, *rent_h, *terms;
+  real *out;
+  AcTypes types;
+  int nrec, ntypes, nsbs;
+};
+
+// 32 threads per (type, receiver) pair, pairs from pair0.  IN_SHARED: run by
+// workgroups of k_ac_shared while others advance u and v, for displacement and
+// pressure only: every displacement term is the tile's, pressure needs 1/M and
+// the partials.
+template <typename real, bool IN_SHARED>
+__device__ __forceinline__ void
+ac_seis_pairs(const AcSeisIn<real> &in, int pair0, real (*s_t)[NPT][2],
+              const int *__restrict__ step_ptr, real dto2) {
+  const int grp = threadIdx.x >> 5, p = threadIdx.x & 31;
+  const int pair = pair0 + grp;
+  const int r = pair % in.nrec, it = pair / in.nrec;
+  const bool active = it < in.ntypes && p < NPT;
+  // the entry's own data is requested before the step counter is known
+  // (all in bounds for every active lane)
+  const int id = r * NPT + p;
+  int j = -1;
+  real t0 = 0, t1 = 0;
+  if (active) {
+    j = in.rent_shared[id];
+    const size_t o = (size_t(it) * in.nrec * NPT + id) * 2;
+    t0 = in.terms[o];
+    t1 = in.terms[o + 1];
+  }
+  const int step = *step_ptr;
+  if (step % in.nsbs != 0)
+    return;
+  const int isig = step / in.nsbs;
+  if (active) {
+    const int type = in.types.t[it & 3];
+    real tx = t0, tz = t1;
+    if (j >= 0 && !(IN_SHARED && type == 0)) {
+      const int g = in.rent_g[id];
+      real f;
+      if (!IN_SHARED && type == 0) {
+        f = in.u[g];
+      } else {
+        // the point's own 1/M and v before its partial sums
+        const real m = in.minv[g];
+        real v = IN_SHARED ? real(0) : in.v[g];
+        real a = ac_shared_sum(in.part, in.shp_off, in.shp_pos, j) * m;
+        v += dto2 * a;
+        f = !IN_SHARED && type == 1 ? v : a;
+      }
+      ac_term(type, f, in.rent_w[2 * id], in.rent_w[2 * id + 1], in.rent_h[id], tx, tz);
+    }
+    s_t[grp][p][0] = tx;
+    s_t[grp][p][1] = tz;
+  }
+  __syncthreads();
+  if (active && p == 0) {
+    real sx = 0, sz = 0;
+    for (int k = 0; k < NPT; ++k) {
+      sx += s_t[grp][k][0];
+      sz += s_t[grp][k][1];
+    }
+    const size_t o = ((size_t(isig) * in.ntypes + it) * in.nrec + r) * 2;
+    in.out[o] = sx;
+    in.out[o + 1] = sz;
+  }
+}
+
+template <typename real>
+__global__ void __launch_bounds__(32 * AC_SEIS_GROUPS)
+    k_ac_seis_fused(AcSeisIn<real> in, const int *__restrict__ step_ptr, real dto2) {
+  __shared__ real s_t[AC_SEIS_GROUPS][NPT][2];
+  ac_seis_pairs<real, false>(in, blockIdx.x * AC_SEIS_GROUPS, s_t, step_ptr, dto2);
+}
+
 // Points shared between tiles: partials summed in tile order, then the same
 // divide / corrector / predictor as the tile's exclusive points.
 template <typename real, int MODE>
@@ -370,8 +453,18 @@ __global__ void __launch_bounds__(AC_NODE_THREADS)
                 const int *__restrict__ shp_off, const int *__restrict__ shp_pos,
                 int nshared, int nex_total, real dt, real dto2, real dt2o2,
                 int *__restrict__ step_ptr, const int *__restrict__ sh_iface,
-                real *__restrict__ chi_dd) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+                real *__restrict__ chi_dd, AcSeisIn<real> seis, int nseis) {
+  // the first nseis workgroups sum the step's seismograms instead
+  int blk = blockIdx.x;
+  if (MODE == AC_STEP && blk < nseis) {
+    __shared__ real s_t[AC_NODE_THREADS / 32][NPT][2];
+    ac_seis_pairs<real, true>(seis, blk * (AC_NODE_THREADS / 32), s_t, step_ptr + 1,
+                              dto2);
+    return;
+  }
+  if (MODE == AC_STEP)
+    blk -= nseis;
+  const int j = blk * blockDim.x + threadIdx.x;
   if (j == 0 && step_ptr && MODE != AC_ASSEMBLE)
     *step_ptr += 1;
   if (j >= nshared)
@@ -406,82 +499,6 @@ __global__ void __launch_bounds__(AC_NODE_THREADS)
   }
 }
 
-// Fused-path seismograms between the tile launch and k_ac_shared: entries on
-// shared points are finished here from the partials (same arithmetic as
-// k_ac_shared); the 25 terms of a receiver are summed in point order.
-template <typename real>
-__global__ void k_ac_seis_fused(const real *__restrict__ U,
-                                const real *__restrict__ V,
-                                const real *__restrict__ Minv,
-                                const real *__restrict__ part,
-                                const int *__restrict__ shp_off,
-                                const int *__restrict__ shp_pos,
-                                const int *__restrict__ rent_g,
-                                const int *__restrict__ rent_shared,
-                                const real *__restrict__ rent_w,
-                                const real *__restrict__ rent_h,
-                                const real *__restrict__ seis_terms, int nrec,
-                                AcTypes types, int ntypes, int nsbs,
-                                const int *__restrict__ step_ptr, real dto2,
-                                real *__restrict__ out) {
-  __shared__ real s_t[AC_SEIS_GROUPS][NPT][2];
-  const int grp = threadIdx.x >> 5, p = threadIdx.x & 31;
-  const int pair = blockIdx.x * AC_SEIS_GROUPS + grp;
-  const int r = pair % nrec, it = pair / nrec;
-  const bool active = it < ntypes && p < NPT;
-  // the entry's own data is requested before the step counter is known
-  // (all in bounds for every active lane)
-  const int id = r * NPT + p;
-  int j = -1, g = 0;
-  real t0 = 0, t1 = 0;
-  if (active) {
-    j = rent_shared[id];
-    g = rent_g[id];
-    const size_t o = (size_t(it) * nrec * NPT + id) * 2;
-    t0 = seis_terms[o];
-    t1 = seis_terms[o + 1];
-  }
-  const int step = *step_ptr;
-  if (step % nsbs != 0)
-    return;
-  const int isig = step / nsbs;
-  if (active) {
-    const int type = types.t[it];
-    real tx, tz;
-    if (j < 0) {
-      tx = t0;
-      tz = t1;
-    } else {
-      real f;
-      if (type == 0) {
-        f = U[g];
-      } else {
-        // the point's own 1/M and v before its partial sums
-        const real m = Minv[g];
-        real v = V[g];
-        real a = ac_shared_sum(part, shp_off, shp_pos, j) * m;
-        v += dto2 * a;
-        f = type == 1 ? v : a;
-      }
-      ac_term(type, f, rent_w[2 * id], rent_w[2 * id + 1], rent_h[id], tx, tz);
-    }
-    s_t[grp][p][0] = tx;
-    s_t[grp][p][1] = tz;
-  }
-  __syncthreads();
-  if (active && p == 0) {
-    real sx = 0, sz = 0;
-    for (int k = 0; k < NPT; ++k) {
-      sx += s_t[grp][k][0];
-      sz += s_t[grp][k][1];
-    }
-    const size_t o = ((size_t(isig) * ntypes + it) * nrec + r) * 2;
-    out[o] = sx;
-    out[o + 1] = sz;
-  }
-}
-
-// Operator-path seismograms from the finished fields.
 template <typename real>
 __global__ void k_ac_seismo(const real *__restrict__ U,
                             const real *__restrict__ V,
@@ -1039,30 +1056,42 @@ private:
         cpl_w_, ue_, cout_li_, cout_k_, chi_dd_, sh_pad_, sh_stride_);
     AC_HIP(hipGetLastError());
   }
-  template <int MODE> void launch_shared(Field &F, int *step_ptr) {
+  // seis: the step's seismogram sums ride in the launch's first workgroups
+  template <int MODE> void launch_shared(Field &F, int *step_ptr, bool seis = false) {
     const HostAssembly2D &A = *asm_;
-    const int n = std::max(1, A.nshared);
-    k_ac_shared<real, MODE><<<dim3((n + AC_NODE_THREADS - 1) / AC_NODE_THREADS),
+    const int n = std::max(1, A.nshared), groups = AC_NODE_THREADS / 32;
+    const int nseis = seis ? (A.nrec * int(A.seis_types.size()) + groups - 1) / groups : 0;
+    k_ac_shared<real, MODE><<<dim3((n + AC_NODE_THREADS - 1) / AC_NODE_THREADS + nseis),
                               dim3(AC_NODE_THREADS), 0, stream_>>>(
         F.u, F.v, F.a, minv_, part_, shp_off_, shp_pos_, A.nshared, A.nex_total,
-        dt_, dto2_, dt2o2_, step_ptr, chi_dd_ ? sh_iface_ : nullptr, chi_dd_);
+        dt_, dto2_, dt2o2_, step_ptr, chi_dd_ ? sh_iface_ : nullptr, chi_dd_,
+        seis_in(F), nseis);
     AC_HIP(hipGetLastError());
   }
+  AcSeisIn<real> seis_in(Field &F) const {
+    const HostAssembly2D &A = *asm_;
+    return {F.u, F.v, minv_, part_, shp_off_, shp_pos_, rent_g_, rent_shared_,
+            rent_w_, rent_h_, seis_terms_, seis_, types_, A.nrec,
+            int(A.seis_types.size()), A.nsbs};
+  }
+  // Displacement and pressure need nothing that k_ac_shared overwrites, so
+  // their sums are workgroups of it on the time steps and not a launch of
+  // their own (4.5 us of the 39 us of a coupled step on 300x200 elements).
   template <int MODE> void fused_step(Field &F) {
     const HostAssembly2D &A = *asm_;
-    const int ntypes = int(A.seis_types.size());
-    const bool seis = A.nrec > 0 && ntypes > 0;
+    const bool seis = A.nrec > 0 && !A.seis_types.empty();
+    bool in_shared = seis && MODE == AC_STEP;
+    for (int t : A.seis_types)
+      in_shared = in_shared && (t == SMX_SEIS_DISPLACEMENT || t == SMX_SEIS_PRESSURE);
     launch_tiles<MODE>(F, 0, step_, seis ? seis_terms_ : nullptr);
-    if (seis) {
-      const int n = A.nrec * ntypes;
+    if (seis && !in_shared) {
+      const int n = A.nrec * int(A.seis_types.size());
       k_ac_seis_fused<real><<<dim3((n + AC_SEIS_GROUPS - 1) / AC_SEIS_GROUPS),
-                              dim3(32 * AC_SEIS_GROUPS), 0, stream_>>>(
-          F.u, F.v, minv_, part_, shp_off_, shp_pos_, rent_g_, rent_shared_,
-          rent_w_, rent_h_, seis_terms_, A.nrec, types_, ntypes, A.nsbs, step_,
-          dto2_, seis_);
+                              dim3(32 * AC_SEIS_GROUPS), 0, stream_>>>(seis_in(F), step_,
+                                                                       dto2_);
       AC_HIP(hipGetLastError());
     }
-    launch_shared<MODE>(F, step_);
+    launch_shared<MODE>(F, step_, in_shared);
   }
   void build_graph(Field &F) {
     if (graph_exec_)

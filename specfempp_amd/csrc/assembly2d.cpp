@@ -1066,11 +1066,12 @@ void assemble2d(const smx_mesh2d &m, const smx_sources2d &src,
   // ---- receiver entries (receiver r, point p) -> entry r*NPT + p.  Entries
   // on a tile's exclusive node are evaluated by that tile; entries on shared
   // nodes by the seismogram pass that runs before the shared-node update,
-  // except when an elastic mesh records displacement (and pressure) only:
-  // the tile that owns the receiver's element has every point's
-  // displacement in hand, so it evaluates all 25 entries.
+  // except when displacement (and pressure) only is recorded: the tile that
+  // owns the receiver's element has every point's displacement (potential)
+  // in hand, so it evaluates all 25 entries.  An acoustic entry on a shared
+  // node keeps the node's index: its pressure is formed from the partials.
   {
-    bool tile_all = !acoustic;
+    bool tile_all = true;
     for (int t : A.seis_types)
       tile_all = tile_all && (t == SMX_SEIS_DISPLACEMENT || t == SMX_SEIS_PRESSURE);
     const int nent = A.nrec * NPT;
@@ -1085,9 +1086,10 @@ void assemble2d(const smx_mesh2d &m, const smx_sources2d &src,
         const int id = r * NPT + p;
         A.rent_g[id] = g;
         A.rent_h[id] = A.rec_h[size_t(r) * NPT + p];
-        if (g >= A.nex_total && !tile_all)
+        const bool shared = g >= A.nex_total;
+        if (shared && (acoustic || !tile_all))
           A.rent_shared[id] = g - A.nex_total;
-        else
+        if (!shared || tile_all)
           ent.push_back({s / ELEM_TILE, A.lidx[size_t(p) * ld + s], id});
       }
     std::stable_sort(ent.begin(), ent.end(),
