@@ -208,9 +208,11 @@ int smx_ctx_create2d(const smx_mesh2d *mesh, const smx_sources2d *sources,
 typedef struct smx_options {
   int tile_elems;  /* elements per tile, 1..64 (default 64) */
   int graph_steps; /* time steps per replayed HIP graph, 1..256 (default 8) */
-  /* 1: tiles re-form per-point geometry from the element control nodes when
-   * the device reproduces every stored value bit for bit (fewer HBM bytes,
-   * more registers); 0 (default): read the stored per-point geometry. */
+  /* 1: check on the device whether the element control nodes reproduce every
+   * stored per-point geometry value bit for bit (smx_ctx_geometry reports
+   * it); 3D tiles then re-form their geometry from them (fewer HBM bytes,
+   * more registers).  2D tiles of 4-node elements always do.  0 (default):
+   * no check, 3D tiles read the stored geometry. */
   int geometry_from_nodes;
   /* Occupancy variant of the FP32 time-step tile kernel of 2D elastic
    * contexts: the fewest waves per SIMD its register allocation must allow

@@ -1127,8 +1127,9 @@ __global__ void __launch_bounds__(NODE3_THREADS)
     st[6 * NPT3] = real(sqrt(double(r) * double(m)));
   } else {
     const float L = k + static_cast<float>(4.0 / 3.0) * m;
-    st[5 * NPT3] = real(sqrtf(L / r) * r);
-    st[6 * NPT3] = real(sqrtf(r * m));
+    // correctly rounded FP32 roots: the double root's rounding is exact
+    st[5 * NPT3] = real(float(sqrt(double(L / r))) * r);
+    st[6 * NPT3] = real(float(sqrt(double(r * m))));
   }
 }
 

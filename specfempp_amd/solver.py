@@ -83,8 +83,9 @@ class Context:
     ``graph_steps`` (time steps per replayed graph) and ``waves_per_eu``
     (occupancy variant of the FP32 time-step tile kernel: 0 default, 6, 7,
     8), as chosen by ``specfempp_amd.autotune``, and ``geometry_from_nodes``
-    (re-form the per-point geometry from the control nodes when the device
-    reproduces it bit for bit; off by default).  ``Context.batch`` builds one
+    (check at set-up whether the device reproduces the stored per-point
+    geometry from the control nodes bit for bit, and report it as
+    ``geometry``; off by default).  ``Context.batch`` builds one
     context over many independent shots."""
 
     def __init__(self, mesh, sources, receivers, dt, nstep, *, nsbs=1,
