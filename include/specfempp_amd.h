@@ -208,11 +208,12 @@ int smx_ctx_create2d(const smx_mesh2d *mesh, const smx_sources2d *sources,
 typedef struct smx_options {
   int tile_elems;  /* elements per tile, 1..64 (default 64) */
   int graph_steps; /* time steps per replayed HIP graph, 1..256 (default 8) */
-  /* 1: check on the device whether the element control nodes reproduce every
-   * stored per-point geometry value bit for bit (smx_ctx_geometry reports
-   * it); 3D tiles then re-form their geometry from them (fewer HBM bytes,
-   * more registers).  2D tiles of 4-node elements always do.  0 (default):
-   * no check, 3D tiles read the stored geometry. */
+  /* 1: check on the device that the element control nodes reproduce every
+   * stored per-point geometry term (smx_ctx_geometry reports it).  A 3D
+   * context then re-forms its geometry from them if they all agree bit for
+   * bit (fewer HBM bytes, more registers).  2D contexts of 4-node elements
+   * always form their geometry from the control nodes, whatever the check
+   * finds.  0 (default): no check, 3D tiles read the stored geometry. */
   int geometry_from_nodes;
   /* Occupancy variant of the FP32 time-step tile kernel of 2D elastic
    * contexts: the fewest waves per SIMD its register allocation must allow
@@ -304,11 +305,15 @@ double smx_ctx_t0(const smx_ctx *ctx);
  * per element instead of one per GLL point; see the assembly's tile flags). */
 int smx_ctx_compact(const smx_ctx *ctx, int *geom_elements, int *mat_elements);
 
-/* Where the stiffness kernels take the geometry from: 0 stored per GLL point,
- * 1 stored per element (affine elements), 2 re-formed on the device from the
- * control nodes with the host's FP32 operations (used only when a set-up
- * check reproduced every stored value bit for bit; `mismatches` counts the
- * values it did not).  A measurement aid with no reference counterpart. */
+/* Where the time-step kernels take the geometry from: 0 stored per GLL point
+ * (2D: 9-node meshes and batches that hold one, per element in tiles of
+ * affine elements), 1 stored per element (3D meshes of affine elements), 2
+ * formed on the device from the control nodes (2D: meshes of 4-node elements,
+ * with the host's FP32 operations but for a corrected quotient; 3D: with the
+ * option geometry_from_nodes where its check passed).  `mismatches`: GLL points
+ * at which that check found a formed term unequal to the stored one (2D
+ * elastic and 3D contexts made with the option; else 0).  A measurement aid
+ * with no reference counterpart. */
 int smx_ctx_geometry(const smx_ctx *ctx, int *mode, long long *mismatches);
 
 /* Mass matrix + Stacey mass term, then its inverse.

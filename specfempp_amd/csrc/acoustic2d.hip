@@ -956,7 +956,7 @@ public:
   }
   void geometry_mode(int *mode, long long *mismatches) const override {
     if (mode)
-      *mode = 0;
+      *mode = stored_ ? 0 : 2;
     if (mismatches)
       *mismatches = 0;
   }

@@ -1355,9 +1355,7 @@ void refresh_compact(HostAssembly2D &A) {
       g = g && A.elem_affine[sl];
       m = m && mat_const[sl];
     }
-    // the geometry source chosen by the solver does not depend on the model
-    A.tiles[t].flags = (g ? TILE_GEOM_ELEM : 0) | (m ? TILE_MAT_ELEM : 0) |
-                       (A.tiles[t].flags & TILE_GEOM_NODES);
+    A.tiles[t].flags = (g ? TILE_GEOM_ELEM : 0) | (m ? TILE_MAT_ELEM : 0);
   }
 }
 

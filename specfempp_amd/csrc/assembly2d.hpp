@@ -67,9 +67,6 @@ struct TileInfo {
 // element-constant lambda+2mu and mu, which they then read per element (mat_e).
 constexpr int32_t TILE_GEOM_ELEM = 1;
 constexpr int32_t TILE_MAT_ELEM = 2;
-// The stored per-point geometry of the tile was found equal, bit for bit, to
-// that of the elements' four control nodes (set by the solver's check).
-constexpr int32_t TILE_GEOM_NODES = 4;
 
 struct HostAssembly2D {
   int nspec = 0, nspec_pad = 0, nglob = 0;

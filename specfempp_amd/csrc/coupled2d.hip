@@ -201,10 +201,7 @@ public:
       *a = 0;
   }
   void geometry_mode(int *mode, long long *mismatches) const override {
-    if (mode)
-      *mode = 0;
-    if (mismatches)
-      *mismatches = 0;
+    el_->geometry_mode(mode, mismatches); // both media have the mesh's elements
   }
 
 private:

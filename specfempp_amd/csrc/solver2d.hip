@@ -61,64 +61,8 @@ using StreamSwap = StreamSwapT<hipStream_t>;
 template <typename real> struct QuadArgs {
   real hp[NGLL][NGLL]; // hp[i][j] = l'_j(xi_i)
   real w[NGLL];
-  float xi[NGLL]; // GLL nodes (FP32, as the host assembly uses them)
-  Q4Deriv d4;     // of 4-node elements at the GLL nodes
+  Q4Deriv d4; // of 4-node elements at the GLL nodes
 };
-
-// The host assembly's per-point geometry of a 4-node element at (xi, gamma),
-// re-formed from its control nodes with the same FP32 operations in the same
-// order and no contraction (shape_function_derivatives2d.cpp:7-20,
-// core/specfem/jacobian/dim2/jacobian.cpp:25-51).  nd points at node 0 of
-// the element's slot in [8][ld] (x0..x3, z0..z3).
-__device__ __forceinline__ void geom_from_nodes2(const float *__restrict__ nd,
-                                                 int ld, float xi, float ga,
-                                                 float &xix, float &xiz,
-                                                 float &gax, float &gaz,
-                                                 float &jac) {
-#pragma clang fp contract(off)
-  const float sp = xi + 1, sm = xi - 1, tp = ga + 1, tm = ga - 1;
-  const float dxi[4] = {0.25f * tm, -0.25f * tm, 0.25f * tp, -0.25f * tp};
-  const float dga[4] = {0.25f * sm, -0.25f * sp, 0.25f * sp, -0.25f * sm};
-  float xxi = 0.0f, zxi = 0.0f, xga = 0.0f, zga = 0.0f;
-#pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const float cx = nd[size_t(n) * ld], cz = nd[size_t(4 + n) * ld];
-    xxi += dxi[n] * cx;
-    zxi += dxi[n] * cz;
-    xga += dga[n] * cx;
-    zga += dga[n] * cz;
-  }
-  jac = xxi * zga - xga * zxi;
-  xix = zga / jac;
-  gax = -zxi / jac;
-  xiz = -xga / jac;
-  gaz = xxi / jac;
-}
-
-// Set-up check: 1 where the re-formed geometry of (point, slot) differs from
-// the stored FP32 value in any bit (slots of padding elements count as equal).
-__global__ void k_geom_check2(const float *__restrict__ nodes,
-                              const float *__restrict__ geom,
-                              const uint8_t *__restrict__ ecolor, int ld,
-                              QuadArgs<float> q,
-                              unsigned char *__restrict__ bad) {
-  const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= long(NPT) * ld)
-    return;
-  const int p = int(t / ld), slot = int(t % ld);
-  if (ecolor[slot] == 0xff) {
-    bad[t] = 0;
-    return;
-  }
-  float g[5];
-  geom_from_nodes2(nodes + slot, ld, q.xi[p % NGLL], q.xi[p / NGLL], g[0],
-                   g[1], g[2], g[3], g[4]);
-  const size_t pld = size_t(NPT) * ld;
-  bool diff = false;
-  for (int c = 0; c < 5; ++c)
-    diff = diff || (__float_as_uint(g[c]) != __float_as_uint(geom[c * pld + t]));
-  bad[t] = diff ? 1 : 0;
-}
 
 template <typename real> struct Vec2;
 template <> struct Vec2<float> {
@@ -295,6 +239,35 @@ template <typename real> struct Prev {
   int *step_next;
   int nex_total;
 };
+
+// ------------------------------------------------------------------------
+// Set-up check: points at which the terms that the steps form from the control
+// nodes (at the element centre in tiles of affine elements) are not the stored
+// FP32 ones; zeros of either sign are equal.
+__global__ void __launch_bounds__(TILE_THREADS)
+    k_geom_check2(const TileInfo *__restrict__ tiles,
+                  const float *__restrict__ nodes, const float *__restrict__ geom,
+                  const float *__restrict__ geom_e, int ld, Q4Deriv d4,
+                  unsigned long long *__restrict__ bad) {
+  const int lane = threadIdx.x & 63, ix = threadIdx.x >> 6;
+  const TileInfo T = tiles[blockIdx.x];
+  if (lane >= T.ecount)
+    return;
+  const size_t slot0 = size_t(blockIdx.x) * ELEM_TILE;
+  const bool centre = (T.flags & TILE_GEOM_ELEM) != 0;
+  ElemColumn<float, false> nodal(nodes, nullptr, size_t(ld), slot0, lane, ix, centre, d4);
+  ElemColumn<float, true> stored(geom, geom_e, size_t(ld), slot0, lane, ix, centre, d4);
+  nodal.open();
+  int n = 0;
+#pragma unroll
+  for (int iz = 0; iz < NGLL; ++iz) {
+    const PointMap<float> f = nodal.at(iz), s = stored.at(iz);
+    n += !(f.xix == s.xix && f.xiz == s.xiz && f.gax == s.gax && f.gaz == s.gaz &&
+           f.jac == s.jac);
+  }
+  if (n)
+    atomicAdd(bad, (unsigned long long)n);
+}
 
 // ------------------------------------------------------------------------
 // Dynamic LDS of k_tile: s_u[nloc_max], s_a[nloc_max] (point displacement and
@@ -1777,7 +1750,6 @@ public:
     quad_.d4 = q4_deriv(A.quad.xi);
     for (int i = 0; i < NGLL; ++i) {
       quad_.w[i] = A.quad.w[i];
-      quad_.xi[i] = A.quad.xi[i];
       for (int j = 0; j < NGLL; ++j)
         quad_.hp[i][j] = A.quad.hprime[i][j];
     }
@@ -2341,7 +2313,7 @@ public:
 
   void geometry_mode(int *mode, long long *mismatches) const override {
     if (mode)
-      *mode = gmode_;
+      *mode = stored_ ? 0 : 2;
     if (mismatches)
       *mismatches = geom_mismatch_;
   }
@@ -2500,44 +2472,21 @@ private:
   }
   long rec_stride() const { return long(n2_ * sizeof(real)); }
 
-  // Checks on the device whether the control nodes reproduce every stored
-  // per-point value bit for bit, and marks the tiles if so.  The steps form
-  // their geometry from the elements' mappings in either case.
+  // Counts the points at which the steps' terms are not the stored ones.
   void check_geometry_from_nodes() {
-    HostAssembly2D &A = *asm_;
-    const int ld = A.nspec_pad;
-    const size_t n = size_t(NPT) * ld;
-    float *gf = nullptr;
-    unsigned char *bad = nullptr;
-    SMX_HIP(hipMalloc(&gf, size_t(5) * n * sizeof(float)));
-    SMX_HIP(hipMalloc(&bad, n));
-    SMX_HIP(hipMemcpyAsync(gf, A.geom.data(), size_t(5) * n * sizeof(float),
-                           hipMemcpyHostToDevice, stream_));
-    QuadArgs<float> qf{};
-    for (int i = 0; i < NGLL; ++i)
-      qf.xi[i] = A.quad.xi[i];
-    k_geom_check2<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream_>>>(
-        nodes_, gf, ecolor_, ld, qf, bad);
+    const HostAssembly2D &A = *asm_;
+    float *g = upload_raw<float>(A.geom), *ge = upload_raw<float>(A.geom_e);
+    auto *bad = upload_raw<unsigned long long>(std::vector<unsigned long long>(1, 0));
+    k_geom_check2<<<dim3(A.ntiles), dim3(TILE_THREADS), 0, stream_>>>(
+        tiles_, nodes_, g, ge, A.nspec_pad, quad_.d4, bad);
     SMX_HIP(hipGetLastError());
-    std::vector<unsigned char> h(n);
-    SMX_HIP(hipMemcpyAsync(h.data(), bad, n, hipMemcpyDeviceToHost, stream_));
+    unsigned long long n = 0;
+    SMX_HIP(hipMemcpyAsync(&n, bad, sizeof n, hipMemcpyDeviceToHost, stream_));
     SMX_HIP(hipStreamSynchronize(stream_));
-    (void)hipFree(gf);
-    (void)hipFree(bad);
-    long long nbad = 0;
-    for (unsigned char b : h)
-      nbad += b;
-    geom_mismatch_ = nbad;
-    if (nbad != 0)
-      return;
-    gmode_ = 2;
-    for (auto &t : A.tiles)
-      if (!(t.flags & TILE_GEOM_ELEM))
-        t.flags |= TILE_GEOM_NODES;
-    SMX_HIP(hipMemcpyAsync(tiles_, A.tiles.data(),
-                           A.tiles.size() * sizeof(TileInfo),
-                           hipMemcpyHostToDevice, stream_));
-    SMX_HIP(hipStreamSynchronize(stream_));
+    geom_mismatch_ = static_cast<long long>(n);
+    release(g);
+    release(ge);
+    release(bad);
   }
 
   // Material arrays on the device.  An FP32 context uses the FP32 values
@@ -2947,7 +2896,6 @@ private:
   real *mat_e_ = nullptr;
   float *nodes_ = nullptr; // 4-node meshes: control nodes
   bool stored_ = false; // the mesh has 9-node elements
-  int gmode_ = 0;
   long long geom_mismatch_ = 0;
   real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *kmr_ = nullptr, *stacey_ = nullptr,
        *src_L_ = nullptr, *stf_ = nullptr, *rent_h_ = nullptr,

@@ -98,8 +98,8 @@ public:
   // Gradient [3][nspec][5][5] (kappa, mu, rho) as double.
   virtual void get_gradient(double *host) = 0;
   virtual void last_adjoint_stats(double *forward_ms, double *adjoint_ms) = 0;
-  // Geometry source of the tile kernels: 0 per point, 1 per element (some
-  // tiles), 2 re-formed from the control nodes; mismatches as in 3D.
+  // Geometry source of the step kernels: 0 stored, 2 formed from the control
+  // nodes; mismatches of the set-up check.
   virtual void geometry_mode(int *mode, long long *mismatches) const = 0;
 
   // Coupled meshes: one solver per medium, driven step by step on the
@@ -127,8 +127,9 @@ template <typename S> struct StreamSwapT {
   ~StreamSwapT() { slot = saved; }
 };
 
-// graph_steps: time steps per replayed HIP graph; nodes_geometry: re-form
-// per-point geometry from the control nodes when bitwise reproducible;
+// graph_steps: time steps per replayed HIP graph; nodes_geometry: check the
+// geometry formed from the control nodes against the stored terms (4-node
+// elastic meshes);
 // waves_per_eu: occupancy variant of the FP32 time-step tile kernel (0 the
 // default, 6, 7 or 8 waves per SIMD; elastic contexts only).
 std::unique_ptr<Solver2DBase> make_solver2d(std::unique_ptr<HostAssembly2D> a,

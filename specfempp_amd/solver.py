@@ -83,10 +83,9 @@ class Context:
     ``graph_steps`` (time steps per replayed graph) and ``waves_per_eu``
     (occupancy variant of the FP32 time-step tile kernel: 0 default, 6, 7,
     8), as chosen by ``specfempp_amd.autotune``, and ``geometry_from_nodes``
-    (check at set-up whether the device reproduces the stored per-point
-    geometry from the control nodes bit for bit, and report it as
-    ``geometry``; off by default).  ``Context.batch`` builds one
-    context over many independent shots."""
+    (check at set-up that the geometry the steps form from the control nodes
+    is the stored one; ``smx_ctx_geometry`` reports it; off by default).
+    ``Context.batch`` builds one context over many independent shots."""
 
     def __init__(self, mesh, sources, receivers, dt, nstep, *, nsbs=1,
                  seismo_types=("displacement",), precision=4, options=None, _batch=None):

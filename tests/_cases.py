@@ -268,6 +268,17 @@ def coupled_box(nx=20, nz=16, h=50.0, nstep=400, dt=1e-3, vertical=True, nrec=8,
                     seismo_types=("displacement", "velocity", "acceleration"))
 
 
+def nine_node_shot(cfg):
+    """A small warped shot of 9-node elements with cfg's time steps and
+    seismograms: a batch that holds it reads every shot's stored geometry."""
+    import dataclasses
+    c = dataclasses.replace(adjoint_small(nx=5, nz=4, nstep=cfg.nstep), dt=cfg.dt,
+                            nsbs=cfg.nsbs, seismo_types=cfg.seismo_types)
+    m = box_mesh(0.0, 250.0, 0.0, 200.0, 5, 4, ngnod=9, absorbing=("bottom", "right", "left"))
+    return warped(dataclasses.replace(c, mesh=dataclasses.replace(
+        m, kappa=c.mesh.kappa, mu=c.mesh.mu, rho=c.mesh.rho)))
+
+
 def warped(cfg, amp=0.18, topo=0.25):
     """cfg with its mesh's control nodes moved smoothly: interior nodes by up
     to ``amp`` element sizes along a sine pattern (edges stay on the box
