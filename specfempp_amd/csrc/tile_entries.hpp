@@ -38,7 +38,12 @@ __device__ __forceinline__ void add_entry_group(int code, F add) {
   for (int r = 0; __any((code >> ENTRY_RANK) >= r); ++r) {
     if ((code >> ENTRY_RANK) == r)
       add(code & ((1 << ENTRY_RANK) - 1));
-    __builtin_amdgcn_wave_barrier(); // rank r's sums before rank r + 1's
+    // rank r's sums before rank r + 1's: the barrier keeps the wavefront's
+    // order of execution, the fences the compiler's order of the accesses
+    // (another lane's sum; within a wavefront they cost no instruction)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 #endif
