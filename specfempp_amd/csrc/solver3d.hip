@@ -45,6 +45,9 @@ namespace {
 
 constexpr int ELEM_THREADS = 128; // >= NPT3 = 125
 constexpr int NODE3_THREADS = 256;
+// elements whose gradient is formed and copied out together: 25 MB of device
+// memory, a grid of 4,000 workgroups
+constexpr int GRAD_ELEMS = 8192;
 constexpr int kGraphSteps3 = 8;
 
 template <typename real> struct Quad3 {
@@ -1213,15 +1216,15 @@ __global__ void __launch_bounds__(NODE3_THREADS)
     bmat[c * nb + j] = real(m[c]);
 }
 
-// d chi / d (kappa, mu, rho) at every point, [3][nspec][125] in mesh element
-// order: wJ and the chain rule in double:
+// d chi / d (kappa, mu, rho) at the n points of consecutive mesh elements,
+// whose slots elem_slot names: wJ and the chain rule in double:
 //   kappa: -wJ Gd,  mu: -wJ (2 Ge - 2/3 Gd),  rho: -wJ (rb . a')_node,
 // plus, at absorbing points, the rho vp / rho vs terms of B and of the
 // Stacey mass, differentiated through rho vp = sqrt(rho (kappa + 4/3 mu))
 // and rho vs = sqrt(rho mu).
 template <typename real>
 __global__ void __launch_bounds__(NODE3_THREADS)
-    k3_gradient_out(const int *__restrict__ slot_elem, const int *__restrict__ ibool,
+    k3_gradient_out(const int *__restrict__ elem_slot, const int *__restrict__ ibool,
                     long n, const int *__restrict__ sslot,
                     const real *__restrict__ stacey, const float *__restrict__ kmr,
                     const float *__restrict__ jac, const real *__restrict__ gd,
@@ -1230,11 +1233,12 @@ __global__ void __launch_bounds__(NODE3_THREADS)
                     const real *__restrict__ d3, long nb, Quad3<float> q,
                     double hdt, double *__restrict__ out) {
 #pragma clang fp contract(off)
-  const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n)
+  const long o = long(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (o >= n)
     return;
-  const long s = i / NPT3;
-  const int p = int(i % NPT3);
+  const long s = elem_slot[o / NPT3];
+  const int p = int(o % NPT3);
+  const long i = s * NPT3 + p;
   const int iz = p / (NGLL * NGLL), iy = (p / NGLL) % NGLL, ix = p % NGLL;
   const int g = ibool[i];
   const double wj = double(q.w[iz]) * q.w[iy] * q.w[ix] * jac[i];
@@ -1272,7 +1276,6 @@ __global__ void __launch_bounds__(NODE3_THREADS)
       gr += dS * m / (2.0 * S);
     }
   }
-  const long o = long(slot_elem[s]) * NPT3 + p;
   out[o] = gk;
   out[n + o] = gm;
   out[2 * n + o] = gr;
@@ -1550,8 +1553,6 @@ public:
     real *mat = A.mat_elem ? mat_el_ : mat_pt_;
     if (mat_ != mat) {
       drop_graph(); // its launches hold the other array
-      if (mat_ != mat_el_ && mat_ != mat_pt_)
-        release(mat_);
       mat_ = mat;
     }
     k3_model_in<real><<<points, NODE3_THREADS, 0, stream_>>>(
@@ -1684,17 +1685,25 @@ public:
     if (!have_gradient_)
       throw SmxError(SMX_ERR_STATE, "no adjoint run");
     const HostAssembly3D &A = *asm_;
-    ensure_model_maps();
-    const long n = long(A.nspec) * NPT3;
+    ensure_point_maps();
+    const size_t all = size_t(A.nspec) * NPT3;
+    const int most = std::min(A.nspec, GRAD_ELEMS);
+    if (!elem_slot_)
+      elem_slot_ = upload<int>(A.elem_slot);
     if (!grad_)
-      grad_ = alloc<double>(3 * size_t(n));
-    k3_gradient_out<real><<<dim3(unsigned((n + NODE3_THREADS - 1) / NODE3_THREADS)),
-                            NODE3_THREADS, 0, stream_>>>(
-        slot_elem_, ibool_, n, sslot_, stacey_, kmr_, jac_, gd_, ge_, racc_, bidx_,
-        t9_, d3_, nbn_alloc_, wq_, 0.5 * double(A.dt), grad_);
-    SMX3_HIP(hipGetLastError());
-    SMX3_HIP(hipMemcpyAsync(out, grad_, 3 * size_t(n) * sizeof(double),
-                            hipMemcpyDeviceToHost, stream_));
+      grad_ = alloc<double>(3 * size_t(most) * NPT3);
+    for (int e = 0; e < A.nspec; e += most) {
+      const long n = long(std::min(most, A.nspec - e)) * NPT3;
+      k3_gradient_out<real><<<dim3(unsigned((n + NODE3_THREADS - 1) / NODE3_THREADS)),
+                              NODE3_THREADS, 0, stream_>>>(
+          elem_slot_ + e, ibool_, n, sslot_, stacey_, kmr_, jac_, gd_, ge_, racc_,
+          bidx_, t9_, d3_, nbn_alloc_, wq_, 0.5 * double(A.dt), grad_);
+      SMX3_HIP(hipGetLastError());
+      for (int c = 0; c < 3; ++c)
+        SMX3_HIP(hipMemcpyAsync(out + c * all + size_t(e) * NPT3, grad_ + c * n,
+                                size_t(n) * sizeof(double), hipMemcpyDeviceToHost,
+                                stream_));
+    }
     SMX3_HIP(hipStreamSynchronize(stream_));
   }
 
@@ -1823,60 +1832,80 @@ private:
     nbn_alloc_ = nb;
   }
 
-  // What the passes over a new model and the gradient read besides the model:
-  // slot order, Jacobians, each node's (slot, point) entries and each absorbing
-  // node's face points, both ascending; and the arrays they write.
-  void ensure_model_maps() {
-    if (slot_elem_)
-      return;
+  // What the gradient and the passes over a new model both read: Jacobians,
+  // the model in slot order (16 B per point).
+  void ensure_point_maps() {
     const HostAssembly3D &A = *asm_;
-    const size_t n = size_t(A.nspec) * NPT3;
-    std::vector<uint32_t> off(size_t(A.nglob) + 1, 0), ent(n);
-    for (size_t i = 0; i < n; ++i)
-      ++off[A.ibool[i] + 1];
-    for (int g = 0; g < A.nglob; ++g)
-      off[g + 1] += off[g];
-    std::vector<uint32_t> at(off.begin(), off.end() - 1);
-    for (size_t i = 0; i < n; ++i)
-      ent[at[A.ibool[i]]++] = uint32_t(i);
-    moff_ = upload<uint32_t>(off);
-    ment_ = upload<uint32_t>(ent);
-    // absorbing nodes are numbered by first touch in ascending order
-    std::vector<int> bidx(size_t(A.nglob), -1);
-    std::vector<std::vector<uint32_t>> points;
-    for (int s = 0; s < A.nspec; ++s) {
-      const int b = A.stacey_slot[s];
-      for (int p = 0; b >= 0 && p < NPT3; ++p) {
-        if (A.stacey[(size_t(b) * 7 + 4) * NPT3 + p] == 0.0f)
-          continue;
-        int &j = bidx[A.ibool[size_t(s) * NPT3 + p]];
-        if (j < 0) {
-          j = int(points.size());
-          points.emplace_back();
-        }
-        points[j].push_back(uint32_t(s) * NPT3 + uint32_t(p));
-      }
-    }
-    std::vector<uint32_t> boff(1, 0), bent;
-    for (const auto &l : points) {
-      bent.insert(bent.end(), l.begin(), l.end());
-      boff.push_back(uint32_t(bent.size()));
-    }
-    nbp_ = uint32_t(bent.size());
-    boff_ = upload<uint32_t>(boff);
-    bent_ = upload<uint32_t>(bent);
-    jac_ = upload<float>(A.jac_pt);
-    kmr_ = upload<float>(A.kappa_mu_rho);
-    model_ = alloc<float>(3 * n);
-    mat_pt_ = alloc<real>(2 * n);
-    mat_el_ = alloc<real>(2 * size_t(A.nspec));
-    flags_ = alloc<int>(2);
     for (int i = 0; i < NGLL; ++i)
       wq_.w[i] = A.quad.w[i];
-    std::vector<int> slot_elem(A.nspec);
-    for (int e = 0; e < A.nspec; ++e)
-      slot_elem[A.elem_slot[e]] = e;
-    slot_elem_ = upload<int>(slot_elem);
+    if (!jac_)
+      jac_ = upload<float>(A.jac_pt);
+    if (!kmr_)
+      kmr_ = upload<float>(A.kappa_mu_rho);
+  }
+
+  // What the passes over a new model read besides it: slot order, each node's
+  // (slot, point) entries and each absorbing node's face points, both
+  // ascending; and the arrays they write.  Every array is made once, also
+  // where an earlier call ran out of memory half-way.
+  void ensure_model_maps() {
+    ensure_point_maps();
+    const HostAssembly3D &A = *asm_;
+    const size_t n = size_t(A.nspec) * NPT3;
+    if (!moff_ || !ment_) {
+      std::vector<uint32_t> off(size_t(A.nglob) + 1, 0), ent(n);
+      for (size_t i = 0; i < n; ++i)
+        ++off[A.ibool[i] + 1];
+      for (int g = 0; g < A.nglob; ++g)
+        off[g + 1] += off[g];
+      std::vector<uint32_t> at(off.begin(), off.end() - 1);
+      for (size_t i = 0; i < n; ++i)
+        ent[at[A.ibool[i]]++] = uint32_t(i);
+      if (!moff_)
+        moff_ = upload<uint32_t>(off);
+      ment_ = upload<uint32_t>(ent);
+    }
+    if (!boff_ || !bent_) {
+      // absorbing nodes are numbered by first touch in ascending order
+      std::vector<int> bidx(size_t(A.nglob), -1);
+      std::vector<std::vector<uint32_t>> points;
+      for (int s = 0; s < A.nspec; ++s) {
+        const int b = A.stacey_slot[s];
+        for (int p = 0; b >= 0 && p < NPT3; ++p) {
+          if (A.stacey[(size_t(b) * 7 + 4) * NPT3 + p] == 0.0f)
+            continue;
+          int &j = bidx[A.ibool[size_t(s) * NPT3 + p]];
+          if (j < 0) {
+            j = int(points.size());
+            points.emplace_back();
+          }
+          points[j].push_back(uint32_t(s) * NPT3 + uint32_t(p));
+        }
+      }
+      std::vector<uint32_t> boff(1, 0), bent;
+      for (const auto &l : points) {
+        bent.insert(bent.end(), l.begin(), l.end());
+        boff.push_back(uint32_t(bent.size()));
+      }
+      nbp_ = uint32_t(bent.size());
+      if (!boff_)
+        boff_ = upload<uint32_t>(boff);
+      bent_ = upload<uint32_t>(bent);
+    }
+    if (!model_)
+      model_ = alloc<float>(3 * n);
+    if (!mat_pt_)
+      mat_pt_ = A.mat_elem ? alloc<real>(2 * n) : mat_;
+    if (!mat_el_)
+      mat_el_ = A.mat_elem ? mat_ : alloc<real>(2 * size_t(A.nspec));
+    if (!flags_)
+      flags_ = alloc<int>(2);
+    if (!slot_elem_) {
+      std::vector<int> slot_elem(A.nspec);
+      for (int e = 0; e < A.nspec; ++e)
+        slot_elem[A.elem_slot[e]] = e;
+      slot_elem_ = upload<int>(slot_elem);
+    }
   }
 
   // Device buffers of the adjoint run (kept between runs).
@@ -2213,8 +2242,8 @@ private:
   // adjoint
   int ckpt_every_ = 0, ckpt_cap_ = 0, rec_every_ = 0, nrin_ = 0;
   long nbn_ = 0, nbn_alloc_ = 1;
-  // device model passes and gradient (ensure_model_maps)
-  int *slot_elem_ = nullptr, *flags_ = nullptr;
+  // gradient (ensure_point_maps) and device model passes (ensure_model_maps)
+  int *elem_slot_ = nullptr, *slot_elem_ = nullptr, *flags_ = nullptr;
   uint32_t *moff_ = nullptr, *ment_ = nullptr, *boff_ = nullptr, *bent_ = nullptr;
   uint32_t nbp_ = 0; // absorbing face points
   float *jac_ = nullptr, *kmr_ = nullptr, *model_ = nullptr;
@@ -2229,7 +2258,7 @@ private:
        *rin_h_ = nullptr;
   hipEvent_t adj_ev_[4] = {};
   bool have_gradient_ = false, have_adj_stats_ = false;
-  double *grad_ = nullptr;
+  double *grad_ = nullptr; // [3] of up to GRAD_ELEMS elements
 };
 
 std::unique_ptr<Solver3DBase> make_solver3d(std::unique_ptr<HostAssembly3D> a,

@@ -66,3 +66,32 @@ def test_rejected_model_changes_nothing():
             ctx.set_model(*bad)
     for a, b in zip(before, _results(ctx)):
         assert np.array_equal(a, b)
+
+
+def test_gradient_memory():
+    """A gradient holds the point maps (16 B per element point) and a bounded
+    output buffer (25 MB), not what a model change needs; a mesh of more than
+    one output piece, against the gradient of a context that made the maps of
+    a model change first."""
+    import torch
+    cfg = adjoint_small3d(n=(32, 24, 22), nstep=32)
+    model = (cfg.mesh.kappa, cfg.mesh.mu, cfg.mesh.rho)
+    print("3D gradient memory: 32x24x22 elements", flush=True)
+    rng = np.random.default_rng(8)
+    gsrc = 1e-9 * rng.standard_normal((cfg.nstep, len(cfg.receivers.x), 3))
+    grads = []
+    for change in (False, True):
+        ctx = _context(cfg, model, 4)
+        if change:
+            ctx.set_model(*model)
+        ctx.run_forward_checkpointed(8)
+        ctx.run_adjoint(gsrc)
+        ctx.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        grads.append(ctx.gradient())
+        held = before - torch.cuda.mem_get_info()[0]
+        # three allocations of 2 MiB granularity beside the sizes
+        assert held <= 16 * 125 * cfg.mesh.nspec + 3 * 8 * 125 * 8192 + (8 << 20), held
+        ctx.close()
+    assert np.abs(grads[0]).max() > 0
+    assert np.array_equal(*grads)
