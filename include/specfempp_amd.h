@@ -414,6 +414,13 @@ int smx_field_device_ptr(smx_ctx *ctx, int field, int which, void **dptr);
 int smx_last_run_stats(smx_ctx *ctx, double *ms, double *stiffness_ms,
                        int *stiffness_launches);
 
+/* Kernel launches of the last smx_run_forward or smx_run_forward_checkpointed
+ * of a 2D elastic context, those inside replayed graphs included (other
+ * contexts: SMX_ERR_STATE).  A time step is one launch where the context's
+ * steps close each other, else two or more.  Measurement aid with no
+ * reference counterpart. */
+int smx_last_run_kernels(const smx_ctx *ctx, int *kernels);
+
 /* Launches the stiffness kernel alone nlaunch times on the context's stream
  * (into a scratch acceleration, leaving the fields untouched) and returns the
  * mean launch duration in ms measured with HIP events.  Measurement aid with

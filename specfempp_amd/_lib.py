@@ -32,7 +32,7 @@ EXPORTS = [
     "smx_ctx_create3d", "smx_ctx_create3d_opts", "smx_ctx_geometry", "smx_ctx_components",
     "smx_update_wavefields_noalloc", "smx_predictor_medium", "smx_corrector_medium",
     "smx_update_wavefields_medium", "smx_ctx_degrees_of_freedom", "smx_set_model_device",
-    "smx_get_gradient_device", "smx_ctx_set_launch",
+    "smx_get_gradient_device", "smx_ctx_set_launch", "smx_last_run_kernels",
 ]
 
 # Medium tags (specfem::element::medium_tag, include/enumerations/medium.hpp:18-28).
@@ -141,6 +141,7 @@ def load():
         "smx_get_ibool": (i, [P, P]),
         "smx_field_device_ptr": (i, [P, i, i, ctypes.POINTER(P)]),
         "smx_last_run_stats": (i, [P, DP, DP, IP]),
+        "smx_last_run_kernels": (i, [P, IP]),
         "smx_time_stiffness": (i, [P, i, DP]),
         "smx_set_model": (i, [P, P, P, P]),
         "smx_run_forward_checkpointed": (i, [P, i]),

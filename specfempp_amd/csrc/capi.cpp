@@ -477,6 +477,13 @@ int smx_last_run_stats(smx_ctx *ctx, double *ms, double *stiffness_ms,
       });
 }
 
+int smx_last_run_kernels(const smx_ctx *ctx, int *kernels) {
+  return guarded([&] {
+    if (!kernels) throw smx::SmxError(SMX_ERR_ARG, "null output");
+    *kernels = S(const_cast<smx_ctx *>(ctx)).last_run_kernels();
+  });
+}
+
 int smx_time_stiffness(smx_ctx *ctx, int nlaunch, double *avg_ms) {
   return guarded([&] {
     auto *s3 = S3(ctx);

@@ -1936,10 +1936,17 @@ public:
       throw SmxError(SMX_ERR_ARG, "steps outside [0, nstep)");
     Field &F = field(SMX_FIELD_FORWARD);
     SMX_HIP(hipEventRecord(ev0_, stream_));
+    launches_ = 0;
     launch_predictor(F);
-    forward_steps(F, istep0, nstep, true);
+    if (chained()) {
+      chain_steps(F, istep0, nstep, true);
+    } else {
+      set_step(istep0);
+      pair_steps(F, nstep, true);
+    }
     SMX_HIP(hipEventRecord(ev1_, stream_));
     last_launches_ = nstep;
+    last_kernels_ = launches_;
     have_stats_ = true;
   }
 
@@ -1955,8 +1962,7 @@ public:
   void enqueue_begin(void *stream, int istep0) override {
     require_init();
     StreamSwap sw(stream_, static_cast<hipStream_t>(stream));
-    k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, istep0);
-    SMX_HIP(hipGetLastError());
+    set_step(istep0);
     launch_predictor(field(SMX_FIELD_FORWARD));
   }
   void enqueue_step(void *stream, bool final) override {
@@ -1991,6 +1997,8 @@ public:
   }
 
   void *field_ptr(int f, int which) override { return pick(f, which); }
+
+  int last_run_kernels() const override { return last_kernels_; }
 
   void last_run_stats(double *ms, double *stiff_ms, int *launches) override {
     float t = 0;
@@ -2160,7 +2168,17 @@ public:
     SMX_HIP(hipEventRecord(adj_ev_[0], stream_));
     for (real *p : {F.u, F.v, F.a}) // from rest
       SMX_HIP(hipMemsetAsync(p, 0, n2_ * sizeof(real), stream_));
+    launches_ = 0;
     launch_predictor(F);
+    // A chain sets its counters and closes its last step in launches of their
+    // own, which pays from three steps a segment on (two where velocity or
+    // acceleration is recorded and a step would be three launches).  80x60
+    // elements, 400 steps, ms, pairs / chains: every step 7.4 / 9.3, every
+    // second 6.7 / 7.1, every third 6.4 / 6.2; with velocity and acceleration
+    // every step 9.0 / 9.7, every second 8.5 / 7.2.
+    const bool chain = chained() && every > (seis_in_tiles_ ? 2 : 1);
+    if (!chain)
+      set_step(0);
     for (int sgm = 0; sgm < nseg; ++sgm) {
       const int k0 = sgm * every, len = std::min(every, A.nstep - k0);
       real *ck = ckpt_ + size_t(sgm) * 2 * n2_;
@@ -2168,8 +2186,12 @@ public:
                              hipMemcpyDeviceToDevice, stream_));
       SMX_HIP(hipMemcpyAsync(ck + n2_, F.v, n2_ * sizeof(real),
                              hipMemcpyDeviceToDevice, stream_));
-      forward_steps(F, k0, len, sgm == nseg - 1);
+      if (chain)
+        chain_steps(F, k0, len, sgm == nseg - 1);
+      else
+        pair_steps(F, len, sgm == nseg - 1);
     }
+    last_kernels_ = launches_;
     SMX_HIP(hipEventRecord(adj_ev_[1], stream_));
     ckpt_every_ = every;
     have_adj_stats_ = false;
@@ -2399,7 +2421,12 @@ private:
   void launch_predictor(Field &F) {
     k_predictor<real><<<node_grid(), dim3(NODE_THREADS), 0, stream_>>>(
         F.u, F.v, F.a, n2_, dt_, dto2_, dt2o2_);
+    launched();
+  }
+  // Checks a kernel launch of the forward path and counts it.
+  void launched() {
     SMX_HIP(hipGetLastError());
+    ++launches_;
   }
 
   // One launch over every tile.  `part` defaults to the context's partials
@@ -2438,7 +2465,7 @@ private:
         A.nspec_pad, A.nstacey_pad, dt_, dto2_, dt2o2_, quad_, rec,
         rec_stride(), std::max(1, rec_every_), cpl_li_, cpl_k_, cpl_w_,
         chi_dd_, sh_pad_, sh_stride_, prev, A.ntiles);
-    SMX_HIP(hipGetLastError());
+    launched();
   }
   void launch_pressure(const real *U, const int *step_ptr, int isig) {
     const HostAssembly2D &A = *asm_;
@@ -2447,7 +2474,7 @@ private:
         U, rent_g_, rent_h_, rec_slot_, geom_, mat_, A.nspec_pad, quad_,
         A.nrec, stypes_, int(A.seis_types.size()), A.nsbs, step_ptr, isig,
         seis_);
-    SMX_HIP(hipGetLastError());
+    launched();
   }
   // seis: the step's seismogram sums in the first workgroup (MODE_STEP with
   // a step counter; every term written by the tiles)
@@ -2468,7 +2495,7 @@ private:
         vs ? vs : V + 2 * size_t(A.nex_total), U, V, Aout, minv_,
         part ? part : part_, shp_off_, shp_pos_, A.nshared, A.nex_total, dt_, dto2_, dt2o2_, step_ptr, rec, rec_stride(),
         std::max(1, rec_every_), ss);
-    SMX_HIP(hipGetLastError());
+    launched();
   }
   long rec_stride() const { return long(n2_ * sizeof(real)); }
 
@@ -2704,7 +2731,7 @@ private:
     const int n = in.nrec * in.ntypes;
     k_seis_fused<real><<<dim3((n + SEIS_GROUPS - 1) / SEIS_GROUPS),
                          dim3(32 * SEIS_GROUPS), 0, stream_>>>(in, step_ptr, dto2_);
-    SMX_HIP(hipGetLastError());
+    launched();
   }
 
   // ---- steps of one launch each.  Launch k of a chain closes step k-1 at the
@@ -2801,33 +2828,40 @@ private:
                                          terms, nullptr, prev, extra);
   }
 
-  // Steps istep0 .. istep0 + n - 1 from the predicted state; final: the last
-  // one stores the corrected v and a, else it predicts the next step.
-  void forward_steps(Field &F, int istep0, int n, bool final) {
+  bool chained() const { return chain_ && !chi_dd_; }
+  void set_step(int istep) {
+    k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, istep);
+    launched();
+  }
+
+  // n steps from the predicted state; final: the last one stores the corrected
+  // v and a, else it predicts the next step.  Of two launches or more each,
+  // from the step that set_step or the call before left:
+  void pair_steps(Field &F, int n, bool final) {
     const int body = final ? n - 1 : n;
-    if (!chain_ || chi_dd_) {
-      k_set_step<<<dim3(1), dim3(64), 0, stream_>>>(step_, istep0);
-      SMX_HIP(hipGetLastError());
-      const int reps = body / gsteps_;
-      if (reps > 0) {
-        build_graph(F, 0);
-        for (int r = 0; r < reps; ++r)
-          SMX_HIP(hipGraphLaunch(graph_exec_[0], stream_));
-      }
-      for (int s = reps * gsteps_; s < body; ++s)
-        fused_step<MODE_STEP>(F);
-      if (final)
-        fused_step<MODE_FINAL>(F);
-      return;
+    const int reps = chained() ? 0 : body / gsteps_; // the graph is a chain's
+    if (reps > 0) {
+      build_graph(F, 0);
+      for (int r = 0; r < reps; ++r)
+        replay(0);
     }
+    for (int s = reps * gsteps_; s < body; ++s)
+      fused_step<MODE_STEP>(F);
+    if (final)
+      fused_step<MODE_FINAL>(F);
+  }
+
+  // of one launch each, from step istep0:
+  void chain_steps(Field &F, int istep0, int n, bool final) {
+    const int body = final ? n - 1 : n;
     k_set_steps<<<dim3(1), dim3(64), 0, stream_>>>(step_ + 4, istep0);
-    SMX_HIP(hipGetLastError());
+    launched();
     int k = 0;
     if (body > 0)
       chain_launch<MODE_STEP>(F, k++);
     while (k > 0 && body - k >= gsteps_) {
       build_graph(F, k & 1);
-      SMX_HIP(hipGraphLaunch(graph_exec_[k & 1], stream_));
+      replay(k & 1);
       k += gsteps_;
     }
     while (k < body)
@@ -2851,12 +2885,19 @@ private:
   // parity q.
   void build_graph(Field &F, int q) {
     capture(graph_[q], graph_exec_[q], stream_, [&] {
+      const int before = launches_;
       for (int s = 0; s < gsteps_; ++s)
-        if (chain_ && !chi_dd_)
+        if (chained())
           chain_launch<MODE_STEP>(F, s + 2 - q);
         else
           fused_step<MODE_STEP>(F);
+      graph_launches_[q] = launches_ - before;
+      launches_ = before;
     });
+  }
+  void replay(int q) {
+    SMX_HIP(hipGraphLaunch(graph_exec_[q], stream_));
+    launches_ += graph_launches_[q];
   }
   // The graphs a run replays: a chain starts its first at k = 1, and meets
   // both parities when gsteps_ is odd.
@@ -2923,6 +2964,8 @@ private:
   bool initialized_ = false, have_stats_ = false;
   double last_stiff_ms_ = 0;
   int last_launches_ = 0;
+  // kernel launches: of the forward calls so far, of each graph, of the last run
+  int launches_ = 0, graph_launches_[2] = {}, last_kernels_ = 0;
   // adjoint: checkpoints [nseg][u, v], the recompute record (every+1 slots
   // of u~, v~, a'), adjoint rb in two parity buffers, gradient accumulators
   real *ckpt_ = nullptr, *rec_[2] = {}, *part_adj_ = nullptr, *rb0_ = nullptr,

@@ -64,6 +64,9 @@ public:
   virtual void get_field(int field, int which, void *host) = 0;
   virtual void set_field(int field, int which, const void *host) = 0;
   virtual void *field_ptr(int field, int which) = 0;
+  virtual int last_run_kernels() const {
+    throw SmxError(SMX_ERR_STATE, "kernel launches are counted for 2D elastic contexts");
+  }
   virtual void last_run_stats(double *ms, double *stiffness_ms,
                               int *stiffness_launches) = 0;
   // Launches only the stiffness kernel n times into a scratch acceleration
