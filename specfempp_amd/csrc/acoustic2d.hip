@@ -112,9 +112,8 @@ __global__ void __launch_bounds__(AC_TILE_THREADS) __attribute__((
               const int *__restrict__ sh_list, const uint16_t *__restrict__ lidx,
               const uint8_t *__restrict__ ecolor, int ncolors,
               const typename ElemColumn<real, STORED>::T *__restrict__ geo,
-           const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
-              const real *__restrict__ mat,
-              const real *__restrict__ mat_e,
+              const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
+              const real *__restrict__ mat, const real *__restrict__ mat_e,
               const int *__restrict__ sslot, const real *__restrict__ stacey,
               const uint32_t *__restrict__ dmask, real *__restrict__ U,
               real *__restrict__ V, real *__restrict__ A,
@@ -499,6 +498,7 @@ __global__ void __launch_bounds__(AC_NODE_THREADS)
   }
 }
 
+// Operator-path seismograms from the finished fields.
 template <typename real>
 __global__ void k_ac_seismo(const real *__restrict__ U,
                             const real *__restrict__ V,
@@ -1043,8 +1043,8 @@ private:
   void launch_tiles_as(Field &F, int istep, int *step_ptr, real *terms,
                        real *part) {
     const HostAssembly2D &A = *asm_;
-    k_ac_tile<real, MODE, STORED><<<dim3(A.ntiles), dim3(AC_TILE_THREADS), lds_bytes_,
-                            stream_>>>(
+    k_ac_tile<real, MODE, STORED><<<dim3(A.ntiles), dim3(AC_TILE_THREADS),
+                                    lds_bytes_, stream_>>>(
         tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors,
         (geometry_source<real, STORED>(nodes_, geom_)),
         (geometry_source<real, STORED>(nodes_, geom_e_)),
@@ -1135,7 +1135,7 @@ private:
       *cout_k_ = nullptr, *sh_iface_ = nullptr, *iface_g_ = nullptr;
   real *cpl_w_ = nullptr, *chi_dd_ = nullptr;
   const real *ue_ = nullptr;
-  real *geom_ = nullptr, *geom_e_ = nullptr,  *mat_ = nullptr, *mat_e_ = nullptr,
+  real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *mat_e_ = nullptr,
        *kmr_ = nullptr, *stacey_ = nullptr, *src_L_ = nullptr, *stf_ = nullptr,
        *rent_h_ = nullptr, *rent_w_ = nullptr, *minv_ = nullptr,
        *part_ = nullptr, *seis_ = nullptr, *seis_terms_ = nullptr,

@@ -42,7 +42,8 @@ __device__ __forceinline__ T &at32(T *base, uint32_t i) {
 
 // The value is formed here: without it the compiler moves a sum's arithmetic
 // past the next barrier and keeps its 10 LDS operands in registers instead of
-// the sum (k_tile: 72 registers and 76 B of spills, 56 and none with it).
+// the sum (k_tile before its element data were requested early: 72 registers
+// and 76 B of spills, 56 and none with it).
 template <typename real> __device__ __forceinline__ void formed(real &x) {
   asm volatile("" : "+v"(x));
 }

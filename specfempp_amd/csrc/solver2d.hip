@@ -288,7 +288,9 @@ __host__ __device__ constexpr size_t tile_lds_bytes(int nloc_max) {
 // STORED: the mesh has 9-node elements, whose geometry is read per point.
 // WPE: if nonzero, the minimum waves per SIMD the compiler must allow (an
 // occupancy variant of the FP32 time-step kernel timed by the autotuner);
-// the arithmetic is the same, only the register allocation changes.
+// the arithmetic is the same, only the register allocation changes (8 waves
+// spill 8 to 28 B a lane; 800x600 elements 103.0, 112.0 and 106.2 us a step at
+// 7, 6 and 8, 400x300 in tiles of 16 74.0 us at 7 and 73.2 at 8).
 // FIN: the launch first closes the step before it at the tile's shared points
 // (every tile that holds a point sums its partials and advances it, with the
 // same result; the point's first tile stores it), which takes the launch of
@@ -302,8 +304,8 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
            const uint8_t *__restrict__ ecolor, int ncolors,
            const typename ElemColumn<real, STORED>::T *__restrict__ geo,
            const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
-           const real *__restrict__ mat,
-           const real *__restrict__ mat_e, const int *__restrict__ sslot, const real *__restrict__ stacey,
+           const real *__restrict__ mat, const real *__restrict__ mat_e,
+           const int *__restrict__ sslot, const real *__restrict__ stacey,
            real *__restrict__ U, real *__restrict__ V, real *__restrict__ A,
            const real *__restrict__ Minv, real *__restrict__ part,
            const int *__restrict__ src_li, const int *__restrict__ src_idx,
@@ -1093,9 +1095,9 @@ __global__ void __launch_bounds__(TILE_THREADS)
                const uint16_t *__restrict__ lidx,
                const uint8_t *__restrict__ ecolor, int ncolors,
                const typename ElemColumn<real, STORED>::T *__restrict__ geo,
-           const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
-           const real *__restrict__ mat,
-               const real *__restrict__ mat_e, const int *__restrict__ sslot, const real *__restrict__ stacey,
+               const typename ElemColumn<real, STORED>::T *__restrict__ geo_e,
+               const real *__restrict__ mat, const real *__restrict__ mat_e,
+               const int *__restrict__ sslot, const real *__restrict__ stacey,
                real *__restrict__ RB0, real *__restrict__ RB1,
                real *__restrict__ UB, real *__restrict__ VB,
                const real *__restrict__ Minv, real *__restrict__ part,
@@ -2493,8 +2495,8 @@ private:
                            dim3(NODE_THREADS), 0, stream_>>>(
         us ? us : U + 2 * size_t(A.nex_total),
         vs ? vs : V + 2 * size_t(A.nex_total), U, V, Aout, minv_,
-        part ? part : part_, shp_off_, shp_pos_, A.nshared, A.nex_total, dt_, dto2_, dt2o2_, step_ptr, rec, rec_stride(),
-        std::max(1, rec_every_), ss);
+        part ? part : part_, shp_off_, shp_pos_, A.nshared, A.nex_total, dt_,
+        dto2_, dt2o2_, step_ptr, rec, rec_stride(), std::max(1, rec_every_), ss);
     launched();
   }
   long rec_stride() const { return long(n2_ * sizeof(real)); }
@@ -2554,11 +2556,10 @@ private:
   void launch_adj_tiles(Field &B, real *rec, hipStream_t st) {
     const HostAssembly2D &A = *asm_;
     k_adj_tile<real, STORED><<<dim3(A.ntiles), dim3(TILE_THREADS), lds_bytes_, st>>>(
-        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors, (geometry_source<real, STORED>(nodes_, geom_)),
+        tiles_, A.nloc_max, sh_list_, lidx_, ecolor_, A.nelem_colors,
+        (geometry_source<real, STORED>(nodes_, geom_)),
         (geometry_source<real, STORED>(nodes_, geom_e_)),
-        mat_, mat_e_, sslot_, stacey_, rb0_, rb1_, B.u, B.v,
-        minv_,
-        part_adj_, rec,
+        mat_, mat_e_, sslot_, stacey_, rb0_, rb1_, B.u, B.v, minv_, part_adj_, rec,
         rec_stride(), rec_every_, bidx_, bsum_, gd_, ge_, racc_, sp_, ss_,
         step_ + 2, A.nspec_pad, A.nstacey_pad, dt_, dto2_, dt2o2_, quad_);
     SMX_HIP(hipGetLastError());
@@ -2746,6 +2747,13 @@ private:
   // one launch against two, 20x15 elements 12.1 / 14.6 us, 160x120 14.4 /
   // 18.8, 320x240 24.1 / 28.3, 680x510 (222 MB) 81.5 / 84.5, but 800x600
   // (307 MB) 117 / 111; with velocity and acceleration 400x300 35.4 / 44.8.
+  // The line is one of the fields' bytes: geometry and moduli stream past in
+  // both forms.  9-node elements with moduli per point (700 B an element) at
+  // 41, 94, 165 and 251 MB of fields 28.8 / 32.2, 44.2 / 46.9, 81.1 / 79.7 and
+  // 128.6 / 129.3, with velocity and acceleration 80.8 / 84.9 and 127.6 /
+  // 132.6 at the last two; 4-node FP64 elements at 83, 147, 194 and 248 MB
+  // 40.0 / 43.4, 61.0 / 63.2, 78.8 / 79.9 and 94.8 / 96.5; 9-node FP64 at 248
+  // MB 141.5 / 139.9, with velocity and acceleration 141.9 / 145.6.
   void setup_chain() {
     const HostAssembly2D &A = *asm_;
     bool four = A.nshared > 0 && A.cpl_li.empty() &&
@@ -2938,8 +2946,8 @@ private:
   float *nodes_ = nullptr; // 4-node meshes: control nodes
   bool stored_ = false; // the mesh has 9-node elements
   long long geom_mismatch_ = 0;
-  real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *kmr_ = nullptr, *stacey_ = nullptr,
-       *src_L_ = nullptr, *stf_ = nullptr, *rent_h_ = nullptr,
+  real *geom_ = nullptr, *geom_e_ = nullptr, *mat_ = nullptr, *kmr_ = nullptr,
+       *stacey_ = nullptr, *src_L_ = nullptr, *stf_ = nullptr, *rent_h_ = nullptr,
        *minv_ = nullptr, *part_ = nullptr, *seis_ = nullptr,
        *seis_terms_ = nullptr, *scratch_u_ = nullptr, *scratch_v_ = nullptr,
        *scratch_part_ = nullptr;

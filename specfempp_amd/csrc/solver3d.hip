@@ -255,8 +255,10 @@ __global__ void __launch_bounds__(RW * ELEM_THREADS)
     s_slot[i] = round_slots[size_t(T.round_off) * RW + i];
   __syncthreads();
   // point sources first, in list order: a source's 125 entries name distinct
-  // points and are added together, one thread each (one thread for the
-  // whole list: 397 instead of 391 us per step of 48^3 elements, 8 sources)
+  // points and are added together, one thread each.  One thread for the whole
+  // list makes the tile wait for its dependent loads one by one: 8^3 elements
+  // 53 us a step with one source and 188 with eight in one element, 36 and 36
+  // this way; 48^3 elements with eight sources apart 393 and 392.
   if (MODE != M3_ASSEMBLE)
     for (int k0 = T.src_off; k0 < T.src_off + T.nsrc; k0 += NPT3) {
       if (tid < NPT3) {
