@@ -205,7 +205,9 @@ def measured_traffic(path=os.path.join(ROOT, "profiles", "k_tile_layered_800x600
 
 def step_bytes(nspec, nglob):
     """Canonical bytes of one time step: u, v, a read + written and M^-1 read
-    once per global point (52 B) plus 800 B per element."""
+    once per global point (52 B) plus 800 B per element (indices, stored
+    geometry and moduli per point).  A measure of the work, of which the steps
+    read less than half: not memory traffic."""
     return 52 * nglob + 800 * nspec
 
 
@@ -692,6 +694,8 @@ def main():
                      "algorithmic_bytes_per_launch": sb, "mean_launch_ms": stiff_ms,
                      "layout": ctx.layout},
         "step_roofline": {"canonical_bytes_per_step": step_bytes(ctx.nspec, ctx.nglob),
+                          "kind": "canonical bytes over time (work, not traffic; "
+                                  "the kernel's own bytes are in roofline)",
                           "achieved_GBs": step_bytes(ctx.nspec, ctx.nglob) * args.steps
                           / wall / 1e9,
                           "frac": step_bytes(ctx.nspec, ctx.nglob) * args.steps / wall / 1e9
