@@ -19,7 +19,7 @@ from specfempp_amd import _lib
 from specfempp_amd.config import Config2D, Receivers2D, Sources2D
 from specfempp_amd.mesh import Mesh2D, box_mesh, elastic_moduli
 from specfempp_amd.solver import Context
-from tests._cases import adjoint_small, rel_l2, warped
+from tests._cases import acoustic_box, adjoint_small, rel_l2, warped
 
 pytestmark = pytest.mark.gpu
 
@@ -128,3 +128,14 @@ def test_point_of_many_tiles(oracle_lib):
     for k in range(3):
         bound = max(1e-5, 2.0 * rel_l2(ref[0][:, k], ref[1][:, k]))
         assert rel_l2(got[0][:, k], ref[0][:, k]) <= bound
+
+
+def test_launch_count_of_other_contexts():
+    print("kernel launches are counted for 2D elastic contexts only", flush=True)
+    cfg = acoustic_box(nx=5, nz=4, nstep=3)
+    ctx = Context(cfg.mesh, cfg.sources, cfg.receivers, cfg.dt, cfg.nstep)
+    n = ctypes.c_int()
+    assert ctx.lib.smx_last_run_kernels(ctx.h, ctypes.byref(n)) == _lib.SMX_ERR_STATE
+    assert ctx.lib.smx_last_run_kernels(None, ctypes.byref(n)) == _lib.SMX_ERR_ARG
+    assert ctx.lib.smx_last_run_kernels(ctx.h, None) == _lib.SMX_ERR_ARG
+    ctx.close()
